@@ -7,6 +7,7 @@
 // L2P; rinv adds the near field (N2N, fmm.hpp:773-809).
 #include "../../include/sfmm.h"
 #include "kernels.hpp"
+#include "m2l_bcast.hpp"
 #include "m2l_dense.hpp"
 #include "tables.hpp"
 #include "tree.hpp"
@@ -16,6 +17,7 @@
 #include <sched.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -40,10 +42,12 @@ int host_threads()
     return std::max(1, n);
 }
 
-// f(begin, end, chunk) over [0, count) cut into `chunks` contiguous ranges, one thread each.
-void parallel_ranges(int64_t count, int chunks, const std::function<void(int64_t, int64_t, int)>& f)
+// f(begin, end, chunk) over [0, count) cut into `chunks` contiguous ranges, one thread each
+// (fewer when a range would be shorter than `least`).
+void parallel_ranges(int64_t count, int chunks, const std::function<void(int64_t, int64_t, int)>& f,
+                     int64_t least = 1024)
 {
-    chunks = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(chunks, count / 1024)));
+    chunks = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(chunks, count / least)));
     if (chunks <= 1) {
         f(0, count, 0);
         return;
@@ -125,9 +129,14 @@ struct DenseHost {
     int op_exp = 0;
 };
 
+struct BcastHost {
+    std::vector<double> rot, coax, az_fwd, az_back;
+};
+
 std::mutex g_tables_mu;
 std::shared_ptr<const sfmm::Tables> g_tables[17];
 std::shared_ptr<const DenseHost> g_dense[17];
+std::shared_ptr<const BcastHost> g_bcast[17];
 
 std::shared_ptr<const sfmm::Tables> tables_for(int p)
 {
@@ -149,6 +158,17 @@ std::shared_ptr<const DenseHost> dense_for(int p, const sfmm::Tables& t)
         g_dense[p] = d;
     }
     return g_dense[p];
+}
+
+std::shared_ptr<const BcastHost> bcast_for(int p, const sfmm::Tables& t)
+{
+    std::lock_guard<std::mutex> lock(g_tables_mu);
+    if (!g_bcast[p]) {
+        auto b = std::make_shared<BcastHost>();
+        sfmm::build_bcast_m2l(t, b->rot, b->coax, b->az_fwd, b->az_back);
+        g_bcast[p] = b;
+    }
+    return g_bcast[p];
 }
 
 }  // namespace
@@ -205,6 +225,11 @@ struct sfmm_plan_s {
     const double* coaxA64 = nullptr;
     const float* rotA32 = nullptr;
     const float* coaxA32 = nullptr;
+    // FP64, p <= kBcastMaxP: M2L with broadcast operators (m2l_bcast.hpp)
+    bool bcast = false;
+    sfmm::BcastArgs bc;                 // operators and azimuths
+    sfmm::BcastArgs bcg[5];             // with the work lists, per component count (built on first use)
+    double* Mx = nullptr;               // its copy of the multipoles
     const double* zero_cols = nullptr;  // 4 (p+1)^2 zeros: M2L columns of absent sources
     const double* m2m_frag = nullptr;   // matrix-core M2M / L2L operators [8][nfrag][64]
     const double* l2l_frag = nullptr;
@@ -233,6 +258,7 @@ struct sfmm_plan_s {
         (void)hipFree(M);
         (void)hipFree(L);
         (void)hipFree(M32);
+        (void)hipFree(Mx);
         (void)hipFree(qbuf);
         (void)hipFree(obuf);
         (void)hipFree(hQ);
@@ -333,8 +359,10 @@ int ensure_buffers(sfmm_plan_s* P, int nc, int qdim)
         (void)hipFree(P->M);
         (void)hipFree(P->L);
         (void)hipFree(P->M32);
+        (void)hipFree(P->Mx);
         P->M = P->L = nullptr;
         P->M32 = nullptr;
+        P->Mx = nullptr;
         P->nc_alloc = 0;
         const size_t bytes = sizeof(double) * static_cast<size_t>(nnode) * nc * P->K;
         if (dev_malloc(&P->M, bytes) != hipSuccess || dev_malloc(&P->L, bytes) != hipSuccess)
@@ -346,6 +374,10 @@ int ensure_buffers(sfmm_plan_s* P, int nc, int qdim)
             const size_t b32 = sizeof(float) * static_cast<size_t>(nnode) * nc * row;
             if (dev_malloc(&P->M32, b32) != hipSuccess) return fail(SFMM_ERR_ALLOC, "hipMalloc failed (FP32 multipoles)");
             HIP_TRY(hipMemset(P->M32, 0, b32));
+        }
+        if (P->bcast) {
+            const size_t bx = sizeof(double) * static_cast<size_t>(nnode + 1) * nc * 2 * sfmm::bcast_pairs(P->p);
+            if (dev_malloc(&P->Mx, bx) != hipSuccess) return fail(SFMM_ERR_ALLOC, "hipMalloc failed (multipole copy)");
         }
         P->nc_alloc = nc;
     }
@@ -553,6 +585,166 @@ int build_m2l_blocks(sfmm_plan_s* P, int nc)
     return SFMM_OK;
 }
 
+// Work of the broadcast M2L: per level and run of 16/nc parents, the four
+// octants of each z half form a group of four rows.  A group's steps go class
+// by class; within a class, step k holds each row's k-th present offset, so a
+// class takes as many steps as its fullest row (full rows of one z half have
+// equal counts: x and y reflections keep the polar class).
+int build_bcast_groups(sfmm_plan_s* P, int nc)
+{
+    if (P->bcg[nc].grp_tgt || P->tree->t.depth < 2) return SFMM_OK;
+    const sfmm::Tree& t = P->tree->t;
+    const int TB = 16 / nc;
+    const auto& cls = P->tables.off_class;
+    const auto& d2 = P->tables.off_d2;
+    const int32_t zero_node = static_cast<int32_t>(P->level_first.back());
+    std::vector<std::vector<int>> class_off(70);
+    for (int off = 0; off < 343; ++off)
+        if (cls[off] >= 0) class_off[cls[off]].push_back(off);
+    struct Grp {
+        int level, half;
+        size_t first;  // index of the rows' first target in their octant lists
+    };
+    std::vector<std::vector<int32_t>> oct_nodes(static_cast<size_t>(8) * (t.depth + 1));
+    std::vector<Grp> groups;
+    for (int l = 2; l <= t.depth; ++l) {
+        const auto& lv = t.lv[l];
+        for (int32_t a = 0; a < lv.n_node(); ++a) oct_nodes[8 * l + (lv.code[a] & 7)].push_back(a);
+        size_t most[2] = {0, 0};
+        for (int o = 0; o < 8; ++o) most[o / 4] = std::max(most[o / 4], oct_nodes[8 * l + o].size());
+        for (size_t b = 0; b < std::max(most[0], most[1]); b += TB)
+            for (int h = 0; h < 2; ++h)
+                if (b < most[h]) groups.push_back({l, h, b});
+    }
+    const int64_t ng = static_cast<int64_t>(groups.size());
+    const int nth = host_threads();
+    // f(off, row, target in row, source) over the interactions of a group's targets
+    auto visit = [&](const Grp& G, auto&& f) {
+        const auto& lv = t.lv[G.level];
+        for (int r = 0; r < 4; ++r) {
+            const auto& nodes = oct_nodes[8 * G.level + 4 * G.half + r];
+            for (int tt = 0; tt < TB && G.first + tt < nodes.size(); ++tt) {
+                const int32_t a = nodes[G.first + tt];
+                for (int64_t k = lv.il_row[a]; k < lv.il_row[a + 1]; ++k) f(int(lv.il_off[k]), r, tt, lv.il_src[k]);
+            }
+        }
+    };
+    std::vector<int64_t> grp_row(static_cast<size_t>(ng) + 1, 0);
+    parallel_ranges(ng, nth, [&](int64_t g0, int64_t g1, int) {
+        std::vector<uint8_t> used(343);
+        for (int64_t g = g0; g < g1; ++g) {
+            std::fill(used.begin(), used.end(), 0);
+            visit(groups[g], [&](int off, int r, int, int32_t) { used[off] |= 1 << r; });
+            int64_t steps = 0;
+            for (const auto& offs : class_off) {
+                int c[4] = {};
+                for (int off : offs)
+                    for (int r = 0; r < 4; ++r) c[r] += used[off] >> r & 1;
+                steps += std::max(std::max(c[0], c[1]), std::max(c[2], c[3]));
+            }
+            grp_row[g + 1] = steps;
+        }
+    }, 32);
+    for (int64_t g = 0; g < ng; ++g) grp_row[g + 1] += grp_row[g];
+    HostArray<int32_t> tgt, meta, src;
+    tgt.resize(static_cast<size_t>(ng) * 4 * TB);
+    meta.resize(static_cast<size_t>(grp_row[ng]) * 4);
+    src.resize(static_cast<size_t>(grp_row[ng]) * 4 * TB);
+    parallel_ranges(ng, nth, [&](int64_t g0, int64_t g1, int) {
+        std::vector<uint8_t> used(343);
+        std::vector<int32_t> cols(static_cast<size_t>(343) * 4 * TB);
+        for (int64_t g = g0; g < g1; ++g) {
+            const Grp& G = groups[g];
+            const int64_t first = P->level_first[G.level];
+            for (int r = 0; r < 4; ++r) {
+                const auto& nodes = oct_nodes[8 * G.level + 4 * G.half + r];
+                for (int tt = 0; tt < TB; ++tt)
+                    tgt[(g * 4 + r) * TB + tt] =
+                        G.first + tt < nodes.size() ? static_cast<int32_t>(first + nodes[G.first + tt]) : -1;
+            }
+            std::fill(used.begin(), used.end(), 0);
+            visit(G, [&](int off, int r, int tt, int32_t s) {
+                int32_t* c = cols.data() + (static_cast<size_t>(off) * 4 + r) * TB;
+                if (!(used[off] >> r & 1)) std::fill(c, c + TB, zero_node);
+                used[off] |= 1 << r;
+                c[tt] = static_cast<int32_t>(first + s);
+            });
+            int64_t st = grp_row[g];
+            for (const auto& offs : class_off) {
+                int64_t steps = 0;
+                for (int r = 0; r < 4; ++r) {
+                    int64_t k = 0;
+                    for (int off : offs) {
+                        if (!(used[off] >> r & 1)) continue;
+                        meta[(st + k) * 4 + r] = off | cls[off] << 9 | d2[off] << 16;
+                        std::copy_n(cols.data() + (static_cast<size_t>(off) * 4 + r) * TB, TB,
+                                    src.data.get() + ((st + k) * 4 + r) * TB);
+                        ++k;
+                    }
+                    steps = std::max(steps, k);
+                }
+                for (int r = 0; r < 4; ++r) {
+                    int64_t k = 0;
+                    for (int off : offs) k += used[off] >> r & 1;
+                    for (; k < steps; ++k) {  // this row has no offset left in the class
+                        meta[(st + k) * 4 + r] = offs[0] | cls[offs[0]] << 9 | d2[offs[0]] << 16;
+                        std::fill_n(src.data.get() + ((st + k) * 4 + r) * TB, TB, zero_node);
+                    }
+                }
+                st += steps;
+            }
+        }
+    }, 32);
+    // workgroups, in launch order (consecutive ones go to the 8 XCDs in turn): the
+    // groups are dealt to the XCDs in contiguous shares of equal steps, so that
+    // neighbours share an L2, and cut into runs towards the end of a share
+    std::vector<int64_t> item, split;
+    std::vector<std::array<int64_t, 4>> share[8];
+    int64_t rows = 0;
+    const int64_t total = grp_row[ng];
+    for (int x = 0; x < 8; ++x) {
+        auto first_at = [&](int64_t step) {  // first group at or after a step
+            return std::lower_bound(grp_row.begin(), grp_row.begin() + ng, step) - grp_row.begin();
+        };
+        const int64_t g0 = x == 0 ? 0 : first_at(total * x / 8), g1 = x == 7 ? ng : first_at(total * (x + 1) / 8);
+        for (int64_t g = g0; g < g1; ++g) {
+            const int64_t r0 = grp_row[g], n = grp_row[g + 1] - r0;
+            const int64_t most = sfmm::bcast_run_steps(P->p, grp_row[g1] - r0, total);
+            const int64_t runs = 2 * n > 3 * most ? (n + most - 1) / most : 1;
+            for (int64_t k = 0; k < runs; ++k)
+                share[x].push_back({g, r0 + n * k / runs, r0 + n * (k + 1) / runs, runs > 1 ? rows + k : -1});
+            if (runs > 1) {
+                split.insert(split.end(), {g, rows, runs});
+                rows += runs;
+            }
+        }
+    }
+    size_t longest = 0;
+    for (const auto& sh : share) longest = std::max(longest, sh.size());
+    for (size_t k = 0; k < longest; ++k)
+        for (const auto& sh : share) {
+            const std::array<int64_t, 4> none{-1, 0, 0, -1};
+            const auto& it = k < sh.size() ? sh[k] : none;
+            item.insert(item.end(), it.begin(), it.end());
+        }
+    sfmm::BcastArgs A = P->bc;
+    A.n_item = static_cast<int64_t>(item.size()) / 4;
+    A.n_split = static_cast<int64_t>(split.size()) / 3;
+    int rc;
+    if ((rc = P->upload(tgt, &A.grp_tgt)) || (rc = P->upload(item, &A.item)) || (rc = P->upload(split, &A.split)) ||
+        (rc = P->upload(meta, &A.step_meta)) || (rc = P->upload(src, &A.step_src)))
+        return rc;
+    if (rows > 0) {
+        void* part = nullptr;
+        if (dev_malloc(&part, sizeof(double) * 64 * P->K * static_cast<size_t>(rows)) != hipSuccess)
+            return fail(SFMM_ERR_ALLOC, "hipMalloc failed (M2L partial sums)");
+        P->owned.push_back(part);
+        A.partial = static_cast<double*>(part);
+    }
+    P->bcg[nc] = A;
+    return SFMM_OK;
+}
+
 // M2M and L2L work lists of every level: blocks of 16/nc parents, each with one
 // entry per child octant present (the children of that octant).  M2M at parent
 // level l and L2L into child level l+1 run over the same blocks.
@@ -633,7 +825,10 @@ int prepare(sfmm_plan_s* P, int kind, int ncharge, int which, sfmm::Mode& mode, 
     HIP_TRY(hipSetDevice(P->device));
     if (int rc = ensure_buffers(P, nc, qdim)) return rc;
     if (P->m2l_kernel == 0) {
-        if (int rc = P->dense ? build_dense_blocks(P, nc) : build_m2l_blocks(P, nc)) return rc;
+        if (int rc = P->dense   ? build_dense_blocks(P, nc)
+                     : P->bcast ? build_bcast_groups(P, nc)
+                                : build_m2l_blocks(P, nc))
+            return rc;
         if (int rc = build_translate_blocks(P, nc)) return rc;
     }
     return SFMM_OK;
@@ -688,7 +883,13 @@ int run_on(sfmm_plan_s* P, sfmm::Mode mode, int nc, int qdim, const double* dQ, 
             sfmm::launch_fp32_copy(P->M + f2 * nc * P->K, P->level_first.back() - f2, nc, P->p, M32 + f2 * nc * row,
                                    P->dense ? P->dense_nodemax + f2 * nc : nullptr, s);
         }
-        if (P->dense) {
+        if (P->bcast) {
+            const int64_t f2 = P->level_first[2], pr = 2 * sfmm::bcast_pairs(P->p);
+            sfmm::launch_pair_copy(P->M + f2 * nc * P->K, P->level_first.back() - f2, nc, P->p, P->Mx + f2 * nc * pr, s);
+            sfmm::BcastArgs A = P->bcg[nc];
+            A.Mx = P->Mx;
+            sfmm::launch_m2l_bcast(A, P->p, nc, P->L, s);
+        } else if (P->dense) {
             sfmm::launch_m2l_dense(P->dns[nc], P->p, nc, M32, P->L, s);
         } else if (P->m2l_kernel == 0) {
             sfmm::M2LArgs& A = P->m2l[nc];
@@ -1381,7 +1582,14 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
         P->dense_ops = dops;
         P->dense_nodemax = const_cast<float*>(dmax);
     }
-    if (!P->dense) {
+    P->bcast = P->precision == SFMM_FP64 && P->m2l_kernel == 0 && p <= sfmm::kBcastMaxP;
+    if (P->bcast) {
+        const std::shared_ptr<const BcastHost> bh = bcast_for(p, tb);
+        if ((rc = P->upload(bh->rot, &P->bc.rot)) || (rc = P->upload(bh->coax, &P->bc.coax)) ||
+            (rc = P->upload(bh->az_fwd, &P->bc.az_fwd)) || (rc = P->upload(bh->az_back, &P->bc.az_back)))
+            return rc;
+    }
+    if (!P->dense && !P->bcast) {
         std::vector<double> rotA, coaxA;
         sfmm::build_m2l_fragments(tb, P->precision == SFMM_MIXED, rotA, coaxA);
         if (P->precision == SFMM_MIXED) {

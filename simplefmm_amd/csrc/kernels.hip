@@ -261,6 +261,31 @@ __global__ __launch_bounds__(64) void p2m_kernel(DevPlan d, int mode, int nc, co
     }
 }
 
+// ------------------------------------------------------------------ pair copy
+// M [node][nc][K] -> [node][pair (n, m)][nc][Re, Im] (m = 0: Re / sqrt 2, Im = 0),
+// plus one node of zeros after the last.
+__global__ __launch_bounds__(256) void pair_copy_kernel(const double* __restrict__ M, int64_t count, int nc, int np,
+                                                        int K, double2* __restrict__ Mx)
+{
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int per = np * nc;
+    const int64_t node = i / per;
+    if (node > count) return;
+    const int k = static_cast<int>(i - node * per);
+    const int pr = k / nc, c = k - pr * nc;
+    int n = static_cast<int>((sqrtf(8.0f * pr + 1.0f) - 1.0f) * 0.5f);
+    while ((n + 1) * (n + 2) / 2 <= pr) ++n;
+    while (n * (n + 1) / 2 > pr) --n;
+    const int m = pr - n * (n + 1) / 2;
+    double2 v{0.0, 0.0};
+    if (node < count) {
+        const double* Mn = M + (node * nc + c) * K;
+        v.x = Mn[rfc(n, m)] * (m == 0 ? 0.70710678118654752 : 1.0);
+        if (m > 0) v.y = Mn[rfs(n, m)];
+    }
+    Mx[i] = v;
+}
+
 // ------------------------------------------------------------------ L2P
 // One thread per particle of the far-field leaves (slot_fleaf maps a sorted
 // slot to its leaf): U_c += (1/w) sum_{n,m} Re(L~ conj R(n,m)), the m > 0
@@ -954,6 +979,14 @@ void launch_p2m(const DevPlan& d, Mode mode, int nc, const double* q, double* M,
     if (d.n_far_leaf == 0) return;
     const int ncq = mode == MODE_POT ? nc : (mode == MODE_CURL ? 3 : 1);
     with_p<P2MRun>(d.p, d, static_cast<int>(mode), ncq, nc, q, M, s);
+}
+
+void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx, hipStream_t s)
+{
+    const int np = (p + 1) * (p + 2) / 2;
+    const int64_t total = (count + 1) * np * nc;
+    hipLaunchKernelGGL(pair_copy_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s, M, count, nc,
+                       np, (p + 1) * (p + 1), reinterpret_cast<double2*>(Mx));
 }
 
 void launch_l2p(const DevPlan& d, int nc, const double* L, double* out, hipStream_t s)

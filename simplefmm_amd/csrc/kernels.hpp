@@ -88,6 +88,25 @@ struct DenseArgs {
     int waves = 8;                      // wavefronts per workgroup (4 or 8): 16 targets per wavefront group
 };
 
+// FP64 M2L with broadcast operators (m2l_bcast.hpp): groups of four rows of 16/nc
+// targets (one level, child octant and run of parents each), walking steps of
+// one polar class with one offset per row and one source per target.
+struct BcastArgs {
+    int64_t n_item = 0;                  // workgroups: groups, or runs of a group's steps
+    const int64_t* item = nullptr;       // [n_item][4] group (-1: none), first step, end, partial row (-1: whole group)
+    int64_t n_split = 0;                 // groups cut into runs
+    const int64_t* split = nullptr;      // [n_split][3] group, first partial row, runs
+    const int32_t* grp_tgt = nullptr;    // [groups][4][16/nc] target gnodes, -1 = none
+    const int32_t* step_meta = nullptr;  // [steps][4] offset id | polar class << 9 | squared distance << 16
+    const int32_t* step_src = nullptr;   // [steps][4][16/nc] source gnodes (absent: the zero node after the last)
+    const double* rot = nullptr;         // [70][registers][16] rotation elements
+    const double* coax = nullptr;        // [28][registers][16] coaxial elements
+    const double* az_fwd = nullptr;      // [343][16] (cos m phi - 1, sin m phi), m = 1..16
+    const double* az_back = nullptr;     // [343][16] (cos m phi, sin m phi)
+    const double* Mx = nullptr;          // multipoles, [gnode][pair (n, m)][nc][Re, Im] (order 0 / sqrt 2) + one zero node
+    double* partial = nullptr;           // [partial rows][(p+1)^2][64]
+};
+
 // Near-field work: items of (leaf, run of its concatenated near sources).
 struct P2PItems {
     int64_t n_item = 0;
@@ -143,6 +162,10 @@ void launch_l2p(const DevPlan& d, int nc, const double* L, double* out, hipStrea
 void launch_m2l_mfma(const M2LArgs& a, int p, int nc, const double* M, double* L, hipStream_t s);
 // p <= 12; M32: the multipoles in FP32, [gnode][nc][dense_order(p).kd] (m2l_dense.hpp)
 void launch_m2l_dense(const DenseArgs& a, int p, int nc, const float* M32, double* L, hipStream_t s);
+// p <= kBcastMaxP (m2l_bcast.hpp).
+void launch_m2l_bcast(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
+// The multipoles of `count` nodes, [nc][(p+1)^2], in the broadcast M2L's order [pair][nc][Re, Im].
+void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx, hipStream_t s);
 // The FP32 copy (F32LayoutOf<p>: the dense M2L's layout for p <= 12, else the
 // real-form order) of `count` nodes of nc x (p+1)^2 FP64 coefficients, with
 // their per-component largest |value| into nodemax when it is not null.

@@ -6,6 +6,7 @@
 // restated here in the level-scaled real form.
 #include "tables.hpp"
 
+#include "m2l_bcast.hpp"
 #include "m2l_dense.hpp"
 #include "m2l_sched.hpp"
 
@@ -215,6 +216,52 @@ void build_m2l_fragments(const Tables& t, bool interleave_rows, std::vector<doub
                 }
             }
     }
+}
+
+void build_bcast_m2l(const Tables& t, std::vector<double>& rot, std::vector<double>& coax, std::vector<double>& az_fwd,
+                     std::vector<double>& az_back)
+{
+    const int P = t.p, NW = bcast_waves(P);
+    const BcastUnits ur = bcast_units(P, false), ut = bcast_units(P, true);
+    const int rr = bcast_reg0(P, ur, false, NW), rt = bcast_reg0(P, ut, true, NW);
+    rot.assign(static_cast<size_t>(70) * rr * 16, 0.0);
+    coax.assign(static_cast<size_t>(28) * rt * 16, 0.0);
+    for (int w = 0; w < NW; ++w) {
+        for (int q = 0; q < ur.count[w]; ++q) {
+            const int n = ur.idx[w][q], part = ur.part[w][q], S = bcast_size(P, false, n, part);
+            const int e0 = bcast_reg0(P, ur, false, w) * 16 + bcast_block(P, ur, false, w, q);
+            for (int cls = 0; cls < 70; ++cls) {
+                const double* src = t.rot.data() + static_cast<size_t>(cls) * 2 * t.rot_size + t.rot_off[n] +
+                                    (part == 0 ? 0 : (n + 1) * (n + 1));
+                double* out = rot.data() + static_cast<size_t>(cls) * rr * 16 + e0;
+                for (int a = 0; a < S; ++a)
+                    for (int b = 0; b < S; ++b) {
+                        const bool a0 = part == 0 && a == 0, b0 = part == 0 && b == 0;
+                        out[b * S + a] = src[a * S + b] * (a0 == b0 ? 1.0 : a0 ? std::sqrt(0.5) : std::sqrt(2.0));
+                    }
+            }
+        }
+        for (int q = 0; q < ut.count[w]; ++q) {
+            const int m = ut.idx[w][q], part = ut.part[w][q], S = bcast_size(P, true, m, part);
+            const int e0 = bcast_reg0(P, ut, true, w) * 16 + bcast_block(P, ut, true, w, q);
+            for (int d2 = 0; d2 < 28; ++d2) {
+                const double* src = t.coax.data() + static_cast<size_t>(d2) * t.coax_size + t.coax_off[m];
+                double* out = coax.data() + static_cast<size_t>(d2) * rt * 16 + e0;
+                for (int a = 0; a < S; ++a)
+                    for (int b = 0; b < S; ++b) out[b * S + a] = src[a * S + b];
+            }
+        }
+    }
+    az_fwd.assign(static_cast<size_t>(343) * 32, 0.0);
+    az_back.assign(static_cast<size_t>(343) * 32, 0.0);
+    for (int off = 0; off < 343; ++off)
+        for (int m = 1; m <= P; ++m) {
+            const double* cs = t.off_cs.data() + (static_cast<size_t>(off) * (P + 1) + m) * 2;
+            const size_t k = static_cast<size_t>(off) * 32 + 2 * (m - 1);
+            az_fwd[k] = cs[0] - 1.0;
+            az_back[k] = cs[0];
+            az_fwd[k + 1] = az_back[k + 1] = cs[1];
+        }
 }
 
 void build_tables(int p, Tables& t)
