@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -1446,11 +1447,29 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
         }
     }
     // ---- near-field work items: a leaf's concatenated near sources cut into runs
-    //      of at most ~2^18 pairs; split leaves go through deterministic partial sums.
+    //      (whole tiles of 64 sources); split leaves go through deterministic partial sums.
     //      Per leaf (host threads): its source count and run length; then the item
     //      and partial-row offsets by prefix sums; then the items in place.
     const int64_t nleaf = static_cast<int64_t>(t.leaf_node.size());
     std::vector<int64_t> near_pref(t.near_begin.size());
+    // A run is one wavefront's work: `most` pairs, a sixteenth of a SIMD's share
+    // of all pairs, so that the last runs end together (an eighth: 200k Plummer
+    // 0.49 ms); a leaf of up to half as much again stays whole (no partial sums).  A source tile takes its latency (LDS, a
+    // tile's fetch) however few targets share it: fewer than 16 count as 16.
+    // (One limit of 2^18 pairs for every tree left a few wavefronts working
+    // alone: 200k Plummer, 1 component, 1.70 -> 0.37 ms; 5k uniform, curl, 172 ->
+    // 24 us; 20k Plummer mixed 460 -> 105 us; 16M Plummer 14.5 -> 13.9 ms.)
+    std::atomic<int64_t> all_pairs{0};
+    parallel_ranges(nleaf, nthreads, [&](int64_t g0, int64_t g1, int) {
+        int64_t sum = 0;
+        for (int64_t g = g0; g < g1; ++g) {
+            int64_t total = 0;
+            for (int64_t r = t.near_row[g]; r < t.near_row[g + 1]; ++r) total += t.near_end[r] - t.near_begin[r];
+            sum += total * std::max<int64_t>(lf_end[g] - lf_begin[g], 16);
+        }
+        all_pairs += sum;
+    });
+    const int64_t most = std::min<int64_t>(int64_t(1) << 18, std::max<int64_t>(1 << 12, all_pairs / (1024 * 16)));
     std::vector<int64_t> l_total(nleaf), l_per(nleaf), l_nitem(nleaf), l_item0(nleaf + 1, 0), l_row0(nleaf + 1, 0),
         l_split0(nleaf + 1, 0);
     parallel_ranges(nleaf, nthreads, [&](int64_t g0, int64_t g1, int) {
@@ -1461,9 +1480,9 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
                 total += t.near_end[r] - t.near_begin[r];
             }
             const int64_t nt = lf_end[g] - lf_begin[g];
-            const int64_t per = std::max<int64_t>(64, ((int64_t(1) << 18) / std::max<int64_t>(nt, 1)) / 64 * 64);
-            l_per[g] = per;
-            l_nitem[g] = std::max<int64_t>(1, (total + per - 1) / per);
+            const int64_t per = std::max<int64_t>(64, most / std::max<int64_t>(nt, 16) / 64 * 64);
+            l_per[g] = total * std::max<int64_t>(nt, 16) * 2 <= 3 * most ? total : per;
+            l_nitem[g] = l_per[g] > 0 ? (total + l_per[g] - 1) / l_per[g] : 1;
             l_total[g] = total;
         }
     });

@@ -811,18 +811,22 @@ __global__ __launch_bounds__(64) void self_correction_kernel(DevPlan d, SelfCorr
     for (int k = 0; k < NOUT; ++k) out[t * NOUT + k] -= a[k];
 }
 
-// Adds the partial sums of split leaves in item order.
-__global__ void p2p_reduce_kernel(DevPlan d, P2PItems w, int nout, const double* __restrict__ partial,
-                                  double* __restrict__ out)
+// Adds the partial sums of split leaves: 16 lanes per target, each over every
+// 16th item, combined in a fixed tree.  (A lone target next to a deep subtree
+// has hundreds of items, one thread's serial loop over them 100 us and more.)
+__global__ __launch_bounds__(256) void p2p_reduce_kernel(DevPlan d, P2PItems w, int nout,
+                                                         const double* __restrict__ partial, double* __restrict__ out)
 {
-    const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t k = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) >> 4;
+    const int l = threadIdx.x & 15;
     if (k >= w.n_split_targets) return;
     const int64_t slot = w.split_slot[k];
     const int64_t first = w.split_first[k], nitem = w.split_nitem[k], stride = w.split_stride[k];
     for (int c = 0; c < nout; ++c) {
         double v = 0.0;
-        for (int64_t i = 0; i < nitem; ++i) v += partial[(first + i * stride) * nout + c];
-        out[slot * nout + c] += v;
+        for (int64_t i = l; i < nitem; i += 16) v += partial[(first + i * stride) * nout + c];
+        for (int h = 8; h > 0; h >>= 1) v += __shfl_xor(v, h, 16);
+        if (l == 0) out[slot * nout + c] += v;
     }
 }
 
@@ -1036,7 +1040,7 @@ void launch_p2p_t(const DevPlan& d, const P2PItems& w, Mode mode, int nc, const 
         }
     }
     if (w.n_split_targets > 0)
-        hipLaunchKernelGGL(p2p_reduce_kernel, dim3(grid_for(w.n_split_targets, 256)), dim3(256), 0, s, d, w, nout,
+        hipLaunchKernelGGL(p2p_reduce_kernel, dim3(grid_for(w.n_split_targets, 16)), dim3(256), 0, s, d, w, nout,
                            partial, out);
 }
 

@@ -122,3 +122,28 @@ def test_mixed_error_against_direct_sum(case):
         assert diff <= bound, k
         assert v <= ref[k] + bound, k
     assert idx.size > 0
+
+
+@pytest.mark.parametrize("prec", [api.FP64, api.MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("lone", [1, 3, 17, 64], ids=str)
+def test_near_field_of_few_targets_beside_many_sources(lone, prec):
+    # a few particles in coarse leaves next to a deep cluster: their near lists
+    # are the whole cluster, cut into many runs, and a tail shorter than a tile
+    rng = np.random.default_rng(lone)
+    n = 30_011
+    pos = np.concatenate([0.499 + 1e-3 * rng.uniform(size=(n - lone, 3)), rng.uniform(0.505, 1.0, (lone, 3))])
+    box = api.Box(corner=[0.0, 0.0, 0.0], width=1.0)
+    part = api.OctreePartitioner(pos, box).refine(20, 64)
+    q = rng.uniform(-1, 1, n)
+    U = np.zeros((n, 4))
+    print(f"lone={lone} prec={prec} depth={part.level()}", flush=True)
+    api.FMM3D(part, 4, ncharge=1, precision=prec).rinv_potgrad(q, U, api.NEAR)
+    for i in list(range(n - lone, n))[:5] + [0, n // 2]:
+        src = part.near_sources(i)
+        src = src[src != i]
+        d = pos[i] - pos[src]
+        r = np.sqrt((d * d).sum(1))
+        ref = np.array([(q[src] / r).sum(), *(-(q[src] / r**3) @ d)])
+        # rounding: sums of |term| times a few units in the last place (FP32 pairs when mixed)
+        scale = np.array([(np.abs(q[src]) / r).sum(), *((np.abs(q[src]) / r**3) @ np.abs(d))])
+        assert np.all(np.abs(U[i] - ref) <= (1e-12 if prec == api.FP64 else 2e-6) * scale)
