@@ -801,6 +801,17 @@ int build_translate_blocks(sfmm_plan_s* P, int nc)
     if ((rc = P->upload(row, &A.blk_row)) || (rc = P->upload(parent_of_block, &A.blk_node)) ||
         (rc = P->upload(oct, &A.ent_oct)) || (rc = P->upload(child, &A.ent_node)))
         return rc;
+    // M2M partial sums of the levels that run split
+    int64_t most = 0;
+    for (int l = 2; l < t.depth; ++l)
+        if (lv_m[l + 1] - lv_m[l] <= sfmm::kTrSplitBlocks) most = std::max(most, lv_m[l + 1] - lv_m[l]);
+    if (most > 0) {
+        void* part = nullptr;
+        if (dev_malloc(&part, sizeof(double) * static_cast<size_t>(most) * 8 * P->K * 16) != hipSuccess)
+            return fail(SFMM_ERR_ALLOC, "hipMalloc failed (M2M partial sums)");
+        P->owned.push_back(part);
+        A.part = static_cast<double*>(part);
+    }
     sfmm::TransArgs B = A;  // published together once every upload succeeded
     A.frag = P->m2m_frag;
     B.frag = P->l2l_frag;
@@ -1469,7 +1480,7 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
         }
         all_pairs += sum;
     });
-    const int64_t most = std::min<int64_t>(int64_t(1) << 18, std::max<int64_t>(1 << 12, all_pairs / (1024 * 16)));
+    const int64_t most = std::min<int64_t>(int64_t(1) << 18, std::max<int64_t>(nleaf >= 4096 ? 1 << 14 : 1 << 12, all_pairs / (1024 * 16)));
     std::vector<int64_t> l_total(nleaf), l_per(nleaf), l_nitem(nleaf), l_item0(nleaf + 1, 0), l_row0(nleaf + 1, 0),
         l_split0(nleaf + 1, 0);
     parallel_ranges(nleaf, nthreads, [&](int64_t g0, int64_t g1, int) {

@@ -149,7 +149,12 @@ struct TransArgs {
     const int32_t* ent_oct = nullptr;   // child octant per entry
     const int32_t* ent_node = nullptr;  // [entries][16/nc] child gnodes, -1 = none
     const double* frag = nullptr;      // [8][nfrag][64]
+    // M2M partial sums of levels of at most kTrSplitBlocks blocks, [block][8][(p+1)^2][16]
+    double* part = nullptr;
 };
+// Levels of at most this many blocks run one workgroup per entry instead of one
+// per block: below it the blocks leave compute units idle.
+constexpr int64_t kTrSplitBlocks = 192;
 
 // All launches are asynchronous on `stream`.
 void launch_gather_charges(const DevPlan& d, int qdim, const double* Q, double* q, hipStream_t s);

@@ -5,12 +5,14 @@ namespace sfmm {
 
 bool translate_lower(const TransArgs& a, LevelSpan b, int p, int nc, double* io, hipStream_t s);
 bool translate_upper(const TransArgs& a, LevelSpan b, int p, int nc, double* io, hipStream_t s);
+bool translate_lower_top(const TransArgs& a, LevelSpan b, int p, int nc, double* io, hipStream_t s);
+bool translate_upper_top(const TransArgs& a, LevelSpan b, int p, int nc, double* io, hipStream_t s);
 
 void launch_translate(const TransArgs& a, LevelSpan blocks, int p, int nc, bool upper, double* io, hipStream_t s)
 {
     if (blocks.count == 0) return;
-    if (upper) translate_upper(a, blocks, p, nc, io, s);
-    else translate_lower(a, blocks, p, nc, io, s);
+    if (upper) (void)(translate_upper(a, blocks, p, nc, io, s) || translate_upper_top(a, blocks, p, nc, io, s));
+    else (void)(translate_lower(a, blocks, p, nc, io, s) || translate_lower_top(a, blocks, p, nc, io, s));
 }
 
 int translate_nfrag(int p, bool upper) { return tr_nfrag(p, upper); }

@@ -45,19 +45,20 @@ __host__ __device__ constexpr int tr_frag(int P, bool upper, int mt)
 }
 __host__ __device__ constexpr int tr_nfrag(int P, bool upper) { return tr_frag(P, upper, tr_mts(P)); }
 
-constexpr int kTrWaves = 4;
+// Wavefronts per workgroup; of the split kernel (small levels) twice as many.
+constexpr int kTrWaves = 4, kTrSplitWaves = 8;
 
 struct TrTiles {
-    int count[kTrWaves] = {};
-    int mt[kTrWaves][24] = {};
+    int count[kTrSplitWaves] = {};
+    int mt[kTrSplitWaves][24] = {};
 };
 
 // m-tiles over the waves: longest k-range first, each to the least loaded wave
-template <int P, bool UPPER>
+template <int P, bool UPPER, int NW>
 __host__ __device__ constexpr TrTiles tr_schedule()
 {
     TrTiles s;
-    int load[kTrWaves] = {};
+    int load[NW] = {};
     bool done[64] = {};
     for (int it = 0; it < tr_mts(P); ++it) {
         int best = -1, cost = -1;
@@ -68,7 +69,7 @@ __host__ __device__ constexpr TrTiles tr_schedule()
             }
         done[best] = true;
         int w = 0;
-        for (int v = 1; v < kTrWaves; ++v)
+        for (int v = 1; v < NW; ++v)
             if (load[v] < load[w]) w = v;
         load[w] += cost;
         s.mt[w][s.count[w]++] = best;
@@ -91,10 +92,10 @@ __device__ __forceinline__ void tr_static_for(F&& f)
 }
 
 // longest k-range among wave W's m-tiles
-template <int P, bool UPPER, int W>
+template <int P, bool UPPER, int W, int NW>
 __host__ __device__ constexpr int tr_maxk()
 {
-    constexpr TrTiles S = tr_schedule<P, UPPER>();
+    constexpr TrTiles S = tr_schedule<P, UPPER, NW>();
     int m = 0;
     for (int q = 0; q < S.count[W]; ++q) {
         const int k = tr_ke(P, UPPER, S.mt[W][q]) - tr_kb(P, UPPER, S.mt[W][q]);
@@ -107,14 +108,16 @@ __host__ __device__ constexpr int tr_maxk()
 // an L2 hit takes several MFMA durations.
 constexpr int kTrDepth = 4;
 
-template <int P, int NC, bool UPPER, int W>
-__device__ __forceinline__ void translate_wave(const TransArgs& a, int64_t blk, double* __restrict__ io, double* Xs)
+// All entries of a block, or (SPLIT) the entry `slot` alone, its M2M result to `part`.
+template <int P, bool UPPER, int W, int NW, bool SPLIT>
+__device__ __forceinline__ void translate_wave(const TransArgs& a, int NC, int64_t blk, int slot,
+                                               double* __restrict__ part, double* __restrict__ io, double* Xs)
 {
     typedef double V4 __attribute__((ext_vector_type(4)));
     constexpr int K = tr_K(P);
-    constexpr int TB = 16 / NC;
+    const int TB = 16 / NC;
     constexpr int NF = tr_nfrag(P, UPPER);
-    constexpr TrTiles S = tr_schedule<P, UPPER>();
+    constexpr TrTiles S = tr_schedule<P, UPPER, NW>();
     constexpr int NT = S.count[W];
     constexpr int NQ = NT > 0 ? NT : 1;
     const int tid = threadIdx.x;
@@ -130,11 +133,11 @@ __device__ __forceinline__ void translate_wave(const TransArgs& a, int64_t blk, 
     // (absent columns read node 0 and are zeroed), so that their latencies
     // overlap.  The first barrier waits for the previous entry's MFMAs.
     auto gather = [&](const int32_t* in) {
-        constexpr int NX = ceil_div(16 * K, 64 * kTrWaves);
+        constexpr int NX = ceil_div(16 * K, 64 * NW);
         double xv[NX];
 #pragma unroll
         for (int j = 0; j < NX; ++j) {
-            const int it = tid + 64 * kTrWaves * j;
+            const int it = tid + 64 * NW * j;
             const int c16 = it / K, r = it - (it / K) * K;
             const int tt = c16 / NC, cc = c16 - (c16 / NC) * NC;
             const bool col_in = it < 16 * K && tt < TB;
@@ -147,14 +150,14 @@ __device__ __forceinline__ void translate_wave(const TransArgs& a, int64_t blk, 
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < NX; ++j) {
-            const int it = tid + 64 * kTrWaves * j;
+            const int it = tid + 64 * NW * j;
             const int c16 = it / K, r = it - (it / K) * K;
             if (it < 16 * K) Xs[r * kTrLdsW + c16] = xv[j];
         }
         __syncthreads();
     };
 
-    constexpr int KM = tr_maxk<P, UPPER, W>();
+    constexpr int KM = tr_maxk<P, UPPER, W, NW>();
     constexpr int DK = kTrDepth;
     double ab[DK][NQ];  // requested fragments: k-step kk of tile q in ab[kk % DK][q]
     // the first k-steps' fragments of octant oct's operator
@@ -192,7 +195,8 @@ __device__ __forceinline__ void translate_wave(const TransArgs& a, int64_t blk, 
         });
     };
 
-    const int64_t e0 = a.blk_row[blk], e1 = a.blk_row[blk + 1];
+    const int64_t b0 = a.blk_row[blk], b1 = a.blk_row[blk + 1];
+    const int64_t e0 = SPLIT ? b0 + slot : b0, e1 = SPLIT ? e0 + 1 : b1;
     if constexpr (UPPER) {
         gather(a.blk_node + blk * TB);  // the parents
         for (int64_t e = e0; e < e1; ++e) {
@@ -229,6 +233,18 @@ __device__ __forceinline__ void translate_wave(const TransArgs& a, int64_t blk, 
             gather(a.ent_node + e * TB);  // the children of the entry's octant
             multiply(A);
         }
+        if constexpr (SPLIT) {  // [row][16 columns]
+            tr_static_for<0, NT>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                constexpr int mt = S.mt[W][q];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 16 * mt + 4 * r + (lane >> 4);
+                    if (row < K) part[row * 16 + col] = acc[q][r];
+                }
+            });
+            return;
+        }
         if (t >= TB) return;
         const int32_t dst = a.blk_node[blk * TB + t];
         if (dst < 0) return;
@@ -254,13 +270,67 @@ __global__ __launch_bounds__(64 * kTrWaves) void translate_kernel(TransArgs a, i
     for (int i = threadIdx.x; i < kTrPad * kTrLdsW; i += 64 * kTrWaves) Xs[K * kTrLdsW + i] = 0.0;
     const int w = threadIdx.x >> 6;
     tr_static_for<0, kTrWaves>([&](auto wc) {
-        if (w == decltype(wc)::value) translate_wave<P, NC, UPPER, decltype(wc)::value>(a, blk, io, Xs);
+        if (w == decltype(wc)::value)
+            translate_wave<P, UPPER, decltype(wc)::value, kTrWaves, false>(a, NC, blk, 0, nullptr, io, Xs);
     });
+}
+
+// Small levels: a workgroup per entry (grid y: the block's entries), so that a
+// level takes one entry's time instead of up to eight in a row.  L2L entries
+// write different children.  M2M entries of a block write partial sums, which
+// translate_sum_kernel adds in entry order (a second launch: handing them to the
+// block's last workgroup takes device-scope fences, 200 us at 128 blocks).
+// p = 12: M2M 30 -> 13 us a level, L2L 38 -> 8; p = 16: 295 -> 50, 300 -> 64.
+template <int P, bool UPPER>
+__global__ __launch_bounds__(64 * kTrSplitWaves) void translate_split_kernel(TransArgs a, int nc, int64_t blk0,
+                                                                            double* __restrict__ io)
+{
+    constexpr int K = tr_K(P);
+    __shared__ double Xs[(K + kTrPad) * kTrLdsW];
+    const int64_t blk = blk0 + blockIdx.x;
+    const int slot = blockIdx.y;
+    if (slot >= a.blk_row[blk + 1] - a.blk_row[blk]) return;
+    for (int i = threadIdx.x; i < kTrPad * kTrLdsW; i += 64 * kTrSplitWaves) Xs[K * kTrLdsW + i] = 0.0;
+    double* part = UPPER ? nullptr : a.part + (static_cast<int64_t>(blockIdx.x) * 8 + slot) * (K * 16);
+    const int w = threadIdx.x >> 6;
+    tr_static_for<0, kTrSplitWaves>([&](auto wc) {
+        if (w == decltype(wc)::value)
+            translate_wave<P, UPPER, decltype(wc)::value, kTrSplitWaves, true>(a, nc, blk, slot, part, io, Xs);
+    });
+}
+
+template <int P>
+__global__ __launch_bounds__(256) void translate_sum_kernel(TransArgs a, int nc, int64_t blk0, int64_t count,
+                                                            double* __restrict__ io)
+{
+    constexpr int K = tr_K(P);
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t b = i / (K * 16);
+    if (b >= count) return;
+    const int k = static_cast<int>(i - b * (K * 16));
+    const int TB = 16 / nc;
+    const int row = k >> 4, col = k & 15;
+    const int t = col / nc, c = col - t * nc;
+    const int32_t dst = t < TB ? a.blk_node[(blk0 + b) * TB + t] : -1;
+    const int n = static_cast<int>(a.blk_row[blk0 + b + 1] - a.blk_row[blk0 + b]);
+    if (dst < 0) return;
+    const double* part = a.part + b * 8 * (K * 16) + k;
+    double v = 0.0;
+    for (int e = 0; e < n; ++e) v += part[e * (K * 16)];
+    io[(static_cast<int64_t>(dst) * nc + c) * K + row] = v;
 }
 
 template <int P, bool UPPER>
 void translate_nc(const TransArgs& a, LevelSpan b, int nc, double* io, hipStream_t s)
 {
+    if (b.count <= kTrSplitBlocks) {
+        hipLaunchKernelGGL((translate_split_kernel<P, UPPER>), dim3(static_cast<unsigned>(b.count), 8),
+                           dim3(64 * kTrSplitWaves), 0, s, a, nc, b.first, io);
+        if constexpr (!UPPER)
+            hipLaunchKernelGGL((translate_sum_kernel<P>), dim3(static_cast<unsigned>((b.count * tr_K(P) * 16 + 255) / 256)),
+                               dim3(256), 0, s, a, nc, b.first, b.count, io);
+        return;
+    }
     const dim3 grid(static_cast<unsigned>(b.count)), blk(64 * kTrWaves);
     switch (nc) {
     case 1: hipLaunchKernelGGL((translate_kernel<P, 1, UPPER>), grid, blk, 0, s, a, b.first, io); break;

@@ -147,3 +147,27 @@ def test_near_field_of_few_targets_beside_many_sources(lone, prec):
         # rounding: sums of |term| times a few units in the last place (FP32 pairs when mixed)
         scale = np.array([(np.abs(q[src]) / r).sum(), *((np.abs(q[src]) / r**3) @ np.abs(d))])
         assert np.all(np.abs(U[i] - ref) <= (1e-12 if prec == api.FP64 else 2e-6) * scale)
+
+
+@pytest.mark.parametrize("p", [3, 12, 16])
+@pytest.mark.parametrize("cells", [1, 768, 769], ids=["one", "last_split", "first_whole"])
+def test_shifts_of_levels_around_the_split(cells, p):
+    # `cells` refined nodes at level 4: 16/nc parents to a block, so 192 or 193
+    # blocks of 4 components, where the M2M and L2L change from a workgroup per
+    # child octant to one per block; children of some octants only
+    rng = np.random.default_rng(cells)
+    at = rng.permutation(16**3)[:cells]
+    corner = np.stack([at // 256, at // 16 % 16, at % 16], 1)
+    sub = rng.uniform(size=(cells, 5, 3))
+    pos = np.concatenate([((corner[:, None, :] + sub) / 16).reshape(-1, 3), rng.uniform(size=(200, 3))])
+    part = api.OctreePartitioner(pos, api.Box(corner=[0.0, 0.0, 0.0], width=1.0)).refine(20, 4)
+    n = len(pos)
+    q = rng.uniform(-1, 1, n)
+    out = []
+    for kernel in (0, 1):
+        print(f"cells={cells} p={p} m2l_kernel={kernel} depth={part.level()}", flush=True)
+        U = np.zeros((n, 4))
+        api.FMM3D(part, p, ncharge=1, m2l_kernel=kernel).rinv_potgrad(q, U, api.FAR)
+        out.append(U)
+    # the same sums in another order: a few thousand terms, 1.1e-16 each
+    assert rel_l2(out[0], out[1]) < 1e-13
