@@ -131,7 +131,7 @@ struct DenseHost {
 };
 
 struct BcastHost {
-    std::vector<double> rot, coax, az_fwd, az_back;
+    std::vector<double> rot, coax, rot_sin, coax_sin, az_fwd, az_back;
 };
 
 std::mutex g_tables_mu;
@@ -166,7 +166,9 @@ std::shared_ptr<const BcastHost> bcast_for(int p, const sfmm::Tables& t)
     std::lock_guard<std::mutex> lock(g_tables_mu);
     if (!g_bcast[p]) {
         auto b = std::make_shared<BcastHost>();
-        sfmm::build_bcast_m2l(t, b->rot, b->coax, b->az_fwd, b->az_back);
+        const bool parted = sfmm::bcast_parted(p);
+        if (parted) sfmm::build_bcast_m2l(t, sfmm::kBcastSin, b->rot_sin, b->coax_sin, b->az_fwd, b->az_back);
+        sfmm::build_bcast_m2l(t, parted ? sfmm::kBcastCos : sfmm::kBcastBoth, b->rot, b->coax, b->az_fwd, b->az_back);
         g_bcast[p] = b;
     }
     return g_bcast[p];
@@ -222,11 +224,9 @@ struct sfmm_plan_s {
     int p2p_tpl = 2;                   // near-field tile shape: targets per lane (1, 2, 4)
     double* p2p_partial = nullptr;     // p2p.n_partial_rows x 4 doubles
     sfmm::M2LArgs m2l[5];              // offset-grouped M2L work per component count (built on first use)
-    const double* rotA64 = nullptr;
-    const double* coaxA64 = nullptr;
     const float* rotA32 = nullptr;
     const float* coaxA32 = nullptr;
-    // FP64, p <= kBcastMaxP: M2L with broadcast operators (m2l_bcast.hpp)
+    // FP64: M2L with broadcast operators (m2l_bcast.hpp)
     bool bcast = false;
     sfmm::BcastArgs bc;                 // operators and azimuths
     sfmm::BcastArgs bcg[5];             // with the work lists, per component count (built on first use)
@@ -577,9 +577,8 @@ int build_m2l_blocks(sfmm_plan_s* P, int nc)
     if ((rc = P->upload(blk_tgt, &A.blk_tgt)) || (rc = P->upload(blk_row, &A.blk_row)) ||
         (rc = P->upload(ent_meta, &A.ent_meta)) || (rc = P->upload(ent_src, &A.ent_src)))
         return rc;
-    A.fp32 = P->precision == SFMM_MIXED;
-    A.rotA = A.fp32 ? static_cast<const void*>(P->rotA32) : static_cast<const void*>(P->rotA64);
-    A.coaxA = A.fp32 ? static_cast<const void*>(P->coaxA32) : static_cast<const void*>(P->coaxA64);
+    A.rotA = P->rotA32;
+    A.coaxA = P->coaxA32;
     A.off_cs = P->d.off_cs;
     A.zero = P->zero_cols;
     P->m2l[nc] = A;
@@ -737,10 +736,12 @@ int build_bcast_groups(sfmm_plan_s* P, int nc)
         return rc;
     if (rows > 0) {
         void* part = nullptr;
-        if (dev_malloc(&part, sizeof(double) * 64 * P->K * static_cast<size_t>(rows)) != hipSuccess)
+        const size_t sums = static_cast<size_t>(rows) * (sfmm::bcast_parted(P->p) ? 2 : 1);
+        if (dev_malloc(&part, sizeof(double) * 64 * P->K * sums) != hipSuccess)
             return fail(SFMM_ERR_ALLOC, "hipMalloc failed (M2L partial sums)");
         P->owned.push_back(part);
         A.partial = static_cast<double*>(part);
+        A.n_partial = rows;
     }
     P->bcg[nc] = A;
     return SFMM_OK;
@@ -875,7 +876,7 @@ int run_on(sfmm_plan_s* P, sfmm::Mode mode, int nc, int qdim, const double* dQ, 
     const bool far = (which & SFMM_FAR) && depth >= 2;  // fmm.hpp:816-820
     // the mixed M2L reads an FP32 copy of the multipoles (levels >= 2), made in
     // one pass before it (P2M and M2M write only the FP64 multipoles)
-    float* M32 = P->m2l_kernel == 0 && (P->dense || P->m2l[nc].fp32) ? P->M32 : nullptr;
+    float* M32 = P->precision == SFMM_MIXED ? P->M32 : nullptr;
     if (far) sfmm::launch_p2m(d, mode, nc, P->qbuf, P->M, s);
     REC(2);
     const sfmm::TransArgs& m2m = P->m2m[nc];
@@ -905,7 +906,7 @@ int run_on(sfmm_plan_s* P, sfmm::Mode mode, int nc, int qdim, const double* dQ, 
             sfmm::launch_m2l_dense(P->dns[nc], P->p, nc, M32, P->L, s);
         } else if (P->m2l_kernel == 0) {
             sfmm::M2LArgs& A = P->m2l[nc];
-            if (A.fp32) A.M32 = P->M32;
+            A.M32 = P->M32;
             sfmm::launch_m2l_mfma(A, P->p, nc, P->M, P->L, s);
         }
         else sfmm::launch_m2l(d, nc, P->M, P->L, s);
@@ -1612,22 +1613,19 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
         P->dense_ops = dops;
         P->dense_nodemax = const_cast<float*>(dmax);
     }
-    P->bcast = P->precision == SFMM_FP64 && P->m2l_kernel == 0 && p <= sfmm::kBcastMaxP;
+    P->bcast = P->precision == SFMM_FP64 && P->m2l_kernel == 0;
     if (P->bcast) {
         const std::shared_ptr<const BcastHost> bh = bcast_for(p, tb);
         if ((rc = P->upload(bh->rot, &P->bc.rot)) || (rc = P->upload(bh->coax, &P->bc.coax)) ||
+            (rc = P->upload(bh->rot_sin, &P->bc.rot_sin)) || (rc = P->upload(bh->coax_sin, &P->bc.coax_sin)) ||
             (rc = P->upload(bh->az_fwd, &P->bc.az_fwd)) || (rc = P->upload(bh->az_back, &P->bc.az_back)))
             return rc;
     }
-    if (!P->dense && !P->bcast) {
+    if (P->precision == SFMM_MIXED && !P->dense) {
         std::vector<double> rotA, coaxA;
-        sfmm::build_m2l_fragments(tb, P->precision == SFMM_MIXED, rotA, coaxA);
-        if (P->precision == SFMM_MIXED) {
-            std::vector<float> r32(rotA.begin(), rotA.end()), c32(coaxA.begin(), coaxA.end());
-            if ((rc = P->upload(r32, &P->rotA32)) || (rc = P->upload(c32, &P->coaxA32))) return rc;
-        } else {
-            if ((rc = P->upload(rotA, &P->rotA64)) || (rc = P->upload(coaxA, &P->coaxA64))) return rc;
-        }
+        sfmm::build_m2l_fragments(tb, true, rotA, coaxA);
+        std::vector<float> r32(rotA.begin(), rotA.end()), c32(coaxA.begin(), coaxA.end());
+        if ((rc = P->upload(r32, &P->rotA32)) || (rc = P->upload(c32, &P->coaxA32))) return rc;
     }
     if ((rc = P->upload(std::vector<double>(4 * P->K, 0.0), &P->zero_cols))) return rc;
     {

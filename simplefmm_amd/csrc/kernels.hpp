@@ -55,7 +55,7 @@ struct DevPlan {
     const double* rec = nullptr;  // recurrence coefficients, see kernels.hip
 };
 
-// Offset-grouped M2L work (see m2l_mfma.hip): blocks of 16/nc targets of one
+// Offset-grouped M2L work of the FP32 pipeline (m2l_mfma.hpp): blocks of 16/nc targets of one
 // level and child octant, each with its list of (offset, 16/nc sources).
 struct M2LArgs {
     int64_t n_block = 0;
@@ -63,12 +63,11 @@ struct M2LArgs {
     const int64_t* blk_row = nullptr;  // [n_block+1] entry ranges
     const int32_t* ent_meta = nullptr; // per entry: offset id | polar class << 9 | distance class << 16
     const int32_t* ent_src = nullptr;  // [entries][16/nc] source gnodes, -1 = none
-    const void* rotA = nullptr;        // rotation fragments [70][2][nfrag][64], double or float
+    const void* rotA = nullptr;        // rotation fragments [70][2][nfrag][64]
     const void* coaxA = nullptr;       // coaxial fragments [28][nfrag][64]
     const double* off_cs = nullptr;    // [343][p+1] (cos, sin) of m * azimuth
     const double* zero = nullptr;      // 4 (p+1)^2 zeros: the columns of absent sources
     const float* M32 = nullptr;        // FP32 copy of the multipoles (FP32 stages gather from it)
-    int fp32 = 0;                      // 1: FP32 MFMA stages (mixed precision)
 };
 
 // Mixed-precision M2L on the f16 matrix cores (m2l_dense.hpp): blocks of
@@ -104,7 +103,9 @@ struct BcastArgs {
     const double* az_fwd = nullptr;      // [343][16] (cos m phi - 1, sin m phi), m = 1..16
     const double* az_back = nullptr;     // [343][16] (cos m phi, sin m phi)
     const double* Mx = nullptr;          // multipoles, [gnode][pair (n, m)][nc][Re, Im] (order 0 / sqrt 2) + one zero node
-    double* partial = nullptr;           // [partial rows][(p+1)^2][64]
+    const double *rot_sin = nullptr, *coax_sin = nullptr;  // p > 13: rot and coax hold the cos blocks, these the sin
+    int64_t n_partial = 0;
+    double* partial = nullptr;           // [n_partial, p > 13: cos then sin][(p+1)^2][64]
 };
 
 // Near-field work: items of (leaf, run of its concatenated near sources).
@@ -167,7 +168,6 @@ void launch_l2p(const DevPlan& d, int nc, const double* L, double* out, hipStrea
 void launch_m2l_mfma(const M2LArgs& a, int p, int nc, const double* M, double* L, hipStream_t s);
 // p <= 12; M32: the multipoles in FP32, [gnode][nc][dense_order(p).kd] (m2l_dense.hpp)
 void launch_m2l_dense(const DenseArgs& a, int p, int nc, const float* M32, double* L, hipStream_t s);
-// p <= kBcastMaxP (m2l_bcast.hpp).
 void launch_m2l_bcast(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
 // The multipoles of `count` nodes, [nc][(p+1)^2], in the broadcast M2L's order [pair][nc][Re, Im].
 void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx, hipStream_t s);

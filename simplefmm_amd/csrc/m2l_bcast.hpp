@@ -33,7 +33,8 @@
 // Measured (M2L stage, before: 16x16x4 MFMA pipeline, 46% matrix-core busy):
 // 16M Plummer p = 12, 4 components 342 -> 175 ms; 2M Plummer 41.2 -> 21.6 ms;
 // 100k uniform p = 8 0.95 -> 0.33 ms; 333k uniform p = 10, 3 components 8.6 ->
-// 3.3 ms; 200k Plummer p = 12, 1 component 1.52 -> 0.91 ms.  Bound by FP64
+// 3.3 ms; 200k Plummer p = 12, 1 component 1.52 -> 0.88 ms; 200k on spheres p = 16
+// (before: one offset at a time, four barriers) 5.03 -> 1.86 ms.  Bound by FP64
 // issue (vector ALU busy 64% of the kernel at p = 12; two wavefronts of a SIMD
 // reach 80%); the rest is waits at the two barriers and for the columns.
 #pragma once
@@ -50,9 +51,24 @@
 
 namespace sfmm {
 
-// Highest order: X fits the LDS (512 (p+1)^2 bytes) and the unrolled stages the
-// instruction cache (24 sum (n+1)^2 + n^2 bytes, 64 KB shared by two CUs).
-constexpr int kBcastMaxP = 13;
+constexpr int kBcastMaxP = 16;
+
+// Which blocks a kernel runs: both parts, or (two kernels, the second adding to
+// the first's result) the cos and the sin blocks.  The parts meet only in the
+// azimuths, so they can run apart; both gather all columns then.  Above p = 13 one
+// kernel for both would exceed the registers and the instruction cache
+// (24 sum (n+1)^2 + n^2 bytes of products; 64 KB shared by two compute units).
+enum BcastPart : int { kBcastBoth = 0, kBcastCos = 1, kBcastSin = 2 };
+SFMM_BC_HD constexpr bool bcast_parted(int P) { return P > 13; }
+SFMM_BC_HD constexpr bool bcast_runs_part(int mode, int part)  // part 0 = cos, 1 = sin
+{
+    return mode == kBcastBoth || mode == (part == 0 ? kBcastCos : kBcastSin);
+}
+// Rows of X.
+SFMM_BC_HD constexpr int bcast_rows(int P, int mode)
+{
+    return mode == kBcastBoth ? (P + 1) * (P + 1) : mode == kBcastCos ? (P + 1) * (P + 2) / 2 : P * (P + 1) / 2;
+}
 
 // Wavefronts per workgroup and, as the register bound, per SIMD: a wavefront's
 // registers hold its share of the operators (2 x 3 sum (n+1)^2 + n^2 doubles /
@@ -88,11 +104,11 @@ SFMM_BC_HD constexpr int bcast_size(int P, bool coax, int i, int part)
 // unless the pair exceeds a wavefront's share by a tenth; longest first, then
 // moves and swaps that lower the largest load of a SIMD (wavefronts w, w + 4, ..),
 // of a wavefront, and its registers for columns.
-SFMM_BC_HD constexpr BcastUnits bcast_units(int P, bool coax)
+SFMM_BC_HD constexpr BcastUnits bcast_units(int P, bool coax, int mode)
 {
     const int NW = bcast_waves(P), NS = NW < 4 ? NW : 4;
     auto cost = [&](int i, int part) {
-        const int s = bcast_size(P, coax, i, part);
+        const int s = bcast_runs_part(mode, part) ? bcast_size(P, coax, i, part) : 0;
         return s == 0 ? 0 : (coax ? s * s + 2 * s : 2 * s * s + 7 * s);
     };
     int total = 0;
@@ -104,9 +120,10 @@ SFMM_BC_HD constexpr BcastUnits bcast_units(int P, bool coax)
     int ni = 0, cols = 0;
     for (int i = 0; i <= P; ++i) {
         const int c0 = cost(i, 0), c1 = cost(i, 1);
-        const bool split = c1 > 0 && 10 * (c0 + c1) * NW > 11 * total;
-        const int nc = bcast_size(P, coax, i, 0);
-        it[ni++] = Item{i, split || c1 == 0 ? 1 : 3, split ? c0 : c0 + c1, nc, 0};
+        const bool split = c0 > 0 && c1 > 0 && 10 * (c0 + c1) * NW > 11 * total;
+        const int nc = bcast_size(P, coax, i, 0), parts = (c0 > 0 ? 1 : 0) | (c1 > 0 ? 2 : 0);
+        if (parts == 0) continue;
+        it[ni++] = Item{i, split ? 1 : parts, split ? c0 : c0 + c1, nc, 0};
         if (split) it[ni++] = Item{i, 2, c1, nc, 0};
         cols += split ? 2 * nc : nc;
     }
@@ -211,7 +228,7 @@ SFMM_BC_HD constexpr int bcast_reg0(int P, const BcastUnits& u, bool coax, int w
 // Workgroups a compute unit holds at once (LDS and wavefronts).
 SFMM_BC_HD constexpr int bcast_resident(int P)
 {
-    const int lds = 160 * 1024 / (512 * (P + 1) * (P + 1)), wv = 4 * bcast_simd_waves(P) / bcast_waves(P);
+    const int lds = 160 * 1024 / (512 * bcast_rows(P, bcast_parted(P) ? kBcastCos : kBcastBoth)), wv = 4 * bcast_simd_waves(P) / bcast_waves(P);
     return lds < wv ? lds : wv;
 }
 

@@ -32,7 +32,12 @@ __device__ __forceinline__ void for_wave(int w, F&& f)
 
 __host__ __device__ constexpr int rc(int n, int m) { return m == 0 ? n * n : n * n + 2 * m - 1; }
 __host__ __device__ constexpr int rs(int n, int m) { return n * n + 2 * m; }
-__host__ __device__ constexpr int row_of(int n, int m, int part) { return part == 0 ? rc(n, m) : rs(n, m); }
+// X row of coefficient (n, m, part)
+__host__ __device__ constexpr int row_of(int mode, int n, int m, int part)
+{
+    return mode == kBcastBoth ? (part == 0 ? rc(n, m) : rs(n, m))
+                              : (part == 0 ? n * (n + 1) / 2 + m : n * (n - 1) / 2 + m - 1);
+}
 
 // c += op[lane LN of this lane's 16-lane row] * x.  The compiler does not form
 // this instruction from v_mov_b64_dpp and v_fma_f64, hence the asm.  A DPP read
@@ -73,8 +78,8 @@ __device__ __forceinline__ void barrier_lds()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int P, bool COAX>
-inline constexpr BcastUnits kUnits = bcast_units(P, COAX);
+template <int P, bool COAX, int MODE>
+inline constexpr BcastUnits kUnits = bcast_units(P, COAX, MODE);
 
 // A stage's work of one wavefront as a list of operator columns (block q, column b).
 struct ColumnList {
@@ -82,11 +87,11 @@ struct ColumnList {
     int q[320] = {};
     int b[320] = {};
 };
-template <int P, bool COAX, int W>
+template <int P, bool COAX, int MODE, int W>
 constexpr ColumnList column_list()
 {
     ColumnList c;
-    const BcastUnits& u = kUnits<P, COAX>;
+    const BcastUnits& u = kUnits<P, COAX, MODE>;
     for (int q = 0; q < u.count[W]; ++q)
         for (int b = 0; b < bcast_size(P, COAX, u.idx[W][q], u.part[W][q]); ++b) {
             c.q[c.n] = q;
@@ -96,20 +101,20 @@ constexpr ColumnList column_list()
     return c;
 }
 
-// Columns read from LDS ahead of their use.
-constexpr int kAheadX = 6;
+// Columns read from LDS ahead of their use (fewer where registers are short).
 
-template <int P, int NC, int W>
+template <int P, int NC, int MODE, int W>
 struct Wave {
     static constexpr int NW = bcast_waves(P);
-    static constexpr const BcastUnits& UR = kUnits<P, false>;
-    static constexpr const BcastUnits& UT = kUnits<P, true>;
+    static constexpr int kAheadX = P >= 16 ? 3 : 6;
+    static constexpr const BcastUnits& UR = kUnits<P, false, MODE>;
+    static constexpr const BcastUnits& UT = kUnits<P, true, MODE>;
     static constexpr int NR = bcast_regs(P, UR, false, W), NT = bcast_regs(P, UT, true, W);
     static constexpr int NB = NR > NT ? NR : NT;
     static constexpr int RR = bcast_reg0(P, UR, false, NW), RT = bcast_reg0(P, UT, true, NW);
     static constexpr int R0 = bcast_reg0(P, UR, false, W), T0 = bcast_reg0(P, UT, true, W);
     static constexpr int NU = UR.count[W], NV = UT.count[W];
-    static constexpr ColumnList CR = column_list<P, false, W>(), CT = column_list<P, true, W>();
+    static constexpr ColumnList CR = column_list<P, false, MODE, W>(), CT = column_list<P, true, MODE, W>();
     // degrees of this wavefront: a degree whose cos and sin blocks are both here
     // appears once in the columns and accumulators
     static constexpr bool first_of(int q)
@@ -159,7 +164,8 @@ struct Wave {
     __device__ __forceinline__ void load_col(const D2* __restrict__ p)
     {
         constexpr Pair pr = pair_of(J);
-        if constexpr (pr.im) col[J] = p[pr.index * NC];
+        if constexpr (MODE == kBcastSin && !pr.im) return;  // order 0 has no sin part
+        else if constexpr (pr.im) col[J] = p[pr.index * NC];
         else col[J].x = p[pr.index * NC].x;
     }
     __device__ __forceinline__ void load_cols(const D2* __restrict__ p)
@@ -195,7 +201,7 @@ struct Wave {
                 constexpr int a = decltype(ac)::value, e = E + b * S + a;
                 if constexpr (b == 0) y[a] = 0.0;
                 fmac_row<e % 16>(y[a], rot.v[e / 16], x[k & 1]);
-                if constexpr (b == S - 1) X[row_of(n, a + part, part) * 64 + lane] = y[a];
+                if constexpr (b == S - 1) X[row_of(MODE, n, a + part, part) * 64 + lane] = y[a];
             });
             __builtin_amdgcn_sched_barrier(0);
         });
@@ -218,7 +224,7 @@ struct Wave {
         auto read = [&](auto kc) {
             constexpr int k = decltype(kc)::value, q = CT.q[k];
             constexpr int m = UT.idx[W][q], part = UT.part[W][q];
-            x[k % kAheadX] = X[row_of(m + CT.b[k], m, part) * 64 + lane];
+            x[k % kAheadX] = X[row_of(MODE, m + CT.b[k], m, part) * 64 + lane];
         };
         static_for<0, (CT.n < kAheadX ? CT.n : kAheadX)>(read);
         static_for<0, CT.n>([&](auto kc) {
@@ -229,7 +235,7 @@ struct Wave {
                 constexpr int a = decltype(ac)::value, e = E + b * S + a;
                 if constexpr (b == 0) y[a] = 0.0;
                 fmac_row<e % 16>(y[a], bank.v[e / 16], x[k % kAheadX]);
-                if constexpr (b == S - 1) X[row_of(m + a, m, part) * 64 + lane] = y[a];
+                if constexpr (b == S - 1) X[row_of(MODE, m + a, m, part) * 64 + lane] = y[a];
             });
             if constexpr (k + kAheadX < CT.n) read(std::integral_constant<int, k + kAheadX>{});
             load_some<LD2 * k / CT.n, LD2*(k + 1) / CT.n>(p);
@@ -246,7 +252,7 @@ struct Wave {
         auto read = [&](auto kc) {
             constexpr int k = decltype(kc)::value, q = CR.q[k];
             constexpr int n = UR.idx[W][q], part = UR.part[W][q];
-            x[k % kAheadX] = X[row_of(n, CR.b[k] + part, part) * 64 + lane];
+            x[k % kAheadX] = X[row_of(MODE, n, CR.b[k] + part, part) * 64 + lane];
         };
         static_for<0, (CR.n < kAheadX ? CR.n : kAheadX)>(read);
         static_for<0, CR.n>([&](auto kc) {
@@ -281,15 +287,28 @@ struct Wave {
     }
 };
 
+// The local expansion that this lane's columns belong to (null: none).
+template <int P, int NC>
+__device__ __forceinline__ double* lane_target(const BcastArgs& a, int64_t g, int lane, double* L)
+{
+    constexpr int TB = 16 / NC;
+    const int l = lane & 15, t = l / NC, c = l - (l / NC) * NC;
+    const int32_t tg = t < TB ? a.grp_tgt[g * (4 * TB) + (lane >> 4) * TB + t] : -1;
+    return tg < 0 ? nullptr : L + (static_cast<int64_t>(tg) * NC + c) * ((P + 1) * (P + 1));
+}
+
 }  // namespace bc
 
-// One workgroup: steps [s0, s1) of a group of four rows; the accumulated
-// columns are left in X ([coefficient][64 lanes]).
-template <int P, int NC, int W>
-__device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t s0, int64_t s1, double* X)
+// One workgroup: steps [s0, s1) of a group of four rows.  The accumulated columns
+// are left in X ([coefficient][64 lanes]) or, where a kernel runs one part (a
+// wavefront's accumulators are then the part's whole result), written: to the
+// run's partial sums, or to the targets' L (sin: added).
+template <int P, int NC, int MODE, int W>
+__device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t g, int64_t s0, int64_t s1, int64_t prow, double* X,
+                                           double* __restrict__ L)
 {
     using namespace bc;
-    using WV = Wave<P, NC, W>;
+    using WV = Wave<P, NC, MODE, W>;
     constexpr int TB = 16 / NC;
     constexpr int NP = bcast_pairs(P);
     const int lane = threadIdx.x & 63;
@@ -356,6 +375,30 @@ __device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t s0, int64
             wn = wnn;
         }
     }
+    if constexpr (MODE != kBcastBoth) {
+        double* part = prow < 0 ? nullptr : a.partial + prow * ((P + 1) * (P + 1) * 64);
+        double* Lt = lane_target<P, NC>(a, g, lane, L);
+        static_for<0, WV::NU>([&](auto qc) {
+            constexpr int n = WV::UR.idx[W][decltype(qc)::value];
+            static_for<(MODE == kBcastSin ? 1 : 0), n + 1>([&](auto mc) {
+                constexpr int m = decltype(mc)::value;
+                constexpr int k = WV::col0(decltype(qc)::value) + m;
+                const double re = m == 0 ? wv.are[k] * 1.4142135623730951 : wv.are[k];
+                if (part) {
+                    part[rc(n, m) * 64 + lane] = re;
+                    if constexpr (m > 0) part[rs(n, m) * 64 + lane] = wv.aim[k];
+                } else if (Lt) {
+                    Lt[rc(n, m)] = MODE == kBcastSin ? Lt[rc(n, m)] + re : re;
+                    if constexpr (m > 0) Lt[rs(n, m)] = MODE == kBcastSin ? Lt[rs(n, m)] + wv.aim[k] : wv.aim[k];
+                }
+            });
+            if constexpr (MODE == kBcastSin)
+                if (part) part[rc(n, 0) * 64 + lane] = 0.0;
+        });
+        if constexpr (MODE == kBcastSin && W == 0)
+            if (part) part[lane] = 0.0;  // degree 0
+        return;
+    } else {
     // accumulators to X rows, order 0 back in the plan's scale: a degree split
     // over two wavefronts adds in two turns
     static_for<0, 2>([&](auto turn) {
@@ -381,36 +424,32 @@ __device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t s0, int64
             }
         });
     });
-    barrier_lds();
+    barrier_lds();    }
 }
 
 // L (or, when the group's steps are cut into several runs, the run's partial
 // sums) written once per target.
-template <int P, int NC>
-__global__ __launch_bounds__(64 * bcast_waves(P), bcast_simd_waves(P)) void m2l_bcast_kernel(BcastArgs a, double* __restrict__ L)
+template <int P, int NC, int MODE>
+__global__ __launch_bounds__(64 * bcast_waves(P), bcast_simd_waves(P)) void m2l_bcast_kernel(BcastArgs a,
+                                                                                            double* __restrict__ L)
 {
     constexpr int NW = bcast_waves(P), NTH = 64 * NW;
     constexpr int K = (P + 1) * (P + 1);
-    constexpr int TB = 16 / NC;
-    __shared__ double X[K * 64];
+    __shared__ double X[bcast_rows(P, MODE) * 64];
     const int64_t* item = a.item + 4 * static_cast<int64_t>(blockIdx.x);
     const int64_t g = item[0], s0 = item[1], s1 = item[2], prow = item[3];
     if (g < 0) return;
     bc::for_wave<0, NW>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), [&](auto wc) {
-        bcast_wave<P, NC, decltype(wc)::value>(a, s0, s1, X);
+        bcast_wave<P, NC, MODE, decltype(wc)::value>(a, g, s0, s1, prow, X, L);
     });
-    if (prow >= 0) {
-        double* part = a.partial + prow * (K * 64);
-        for (int i = threadIdx.x; i < K * 64; i += NTH) part[i] = X[i];
-        return;
+    if constexpr (MODE == kBcastBoth) {
+        if (prow >= 0) {
+            double* part = a.partial + prow * (K * 64);
+            for (int i = threadIdx.x; i < K * 64; i += NTH) part[i] = X[i];
+        } else if (double* Lt = bc::lane_target<P, NC>(a, g, threadIdx.x & 63, L)) {
+            for (int r = threadIdx.x >> 6; r < K; r += NW) Lt[r] = X[r * 64 + (threadIdx.x & 63)];
+        }
     }
-    const int lane = threadIdx.x & 63;
-    const int l = lane & 15, t = l / NC, c = l - (l / NC) * NC;
-    if (t >= TB) return;
-    const int32_t tg = a.grp_tgt[g * (4 * TB) + (lane >> 4) * TB + t];
-    if (tg < 0) return;
-    double* Lt = L + (static_cast<int64_t>(tg) * NC + c) * K;
-    for (int r = threadIdx.x >> 6; r < K; r += NW) Lt[r] = X[r * 64 + lane];
 }
 
 // L from the partial sums of a group's runs, added in run order.
@@ -432,13 +471,27 @@ __global__ __launch_bounds__(256) void m2l_bcast_reduce_kernel(BcastArgs a, doub
     const int n = static_cast<int>(a.split[3 * q + 2]);
     double v = 0.0;
     for (int run = 0; run < n; ++run) v += p[static_cast<int64_t>(run) * (K * 64)];
+    if constexpr (bcast_parted(P)) {
+        p += a.n_partial * (K * 64);
+        for (int run = 0; run < n; ++run) v += p[static_cast<int64_t>(run) * (K * 64)];
+    }
     L[(static_cast<int64_t>(tg) * NC + c) * K + r] = v;
 }
 
 template <int P, int NC>
 void bcast_launch(const BcastArgs& a, double* L, hipStream_t s)
 {
-    hipLaunchKernelGGL((m2l_bcast_kernel<P, NC>), dim3(static_cast<unsigned>(a.n_item)), dim3(64 * bcast_waves(P)), 0, s, a, L);
+    const dim3 grid(static_cast<unsigned>(a.n_item)), blk(64 * bcast_waves(P));
+    if constexpr (bcast_parted(P)) {
+        hipLaunchKernelGGL((m2l_bcast_kernel<P, NC, kBcastCos>), grid, blk, 0, s, a, L);
+        BcastArgs b = a;  // the sin part's operators and partial sums
+        b.rot = a.rot_sin;
+        b.coax = a.coax_sin;
+        if (a.n_split > 0) b.partial += a.n_partial * ((P + 1) * (P + 1) * 64);
+        hipLaunchKernelGGL((m2l_bcast_kernel<P, NC, kBcastSin>), grid, blk, 0, s, b, L);
+    } else {
+        hipLaunchKernelGGL((m2l_bcast_kernel<P, NC, kBcastBoth>), grid, blk, 0, s, a, L);
+    }
     if (a.n_split > 0) {
         const int64_t n = a.n_split * (P + 1) * (P + 1) * 64;
         hipLaunchKernelGGL((m2l_bcast_reduce_kernel<P, NC>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,

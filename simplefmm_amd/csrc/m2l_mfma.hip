@@ -6,24 +6,23 @@ namespace sfmm {
 void launch_m2l_mfma(const M2LArgs& a, int p, int nc, const double* M, double* L, hipStream_t s)
 {
     if (a.n_block == 0) return;
-    if (a.fp32) {
-        // orders 13..16; the mixed path of lower orders runs m2l_dense.hpp
-        (void)m2l_f32_top(a, p, nc, M, L, s);
-    } else {
-        // orders 14..16; FP64 of lower orders runs m2l_bcast.hpp
-        (void)m2l_f64_top(a, p, nc, M, L, s);
-    }
+    // orders 13..16; the mixed path of lower orders runs m2l_dense.hpp
+    (void)m2l_f32_top(a, p, nc, M, L, s);
 }
 
 // one translation unit per order range keeps the builds parallel
 bool m2l_bcast_lo(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
 bool m2l_bcast_hi(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
 bool m2l_bcast_top(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
+bool m2l_bcast_14(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
+bool m2l_bcast_15(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
+bool m2l_bcast_16(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
 
 void launch_m2l_bcast(const BcastArgs& a, int p, int nc, double* L, hipStream_t s)
 {
     if (a.n_item == 0) return;
-    if (!m2l_bcast_lo(a, p, nc, L, s) && !m2l_bcast_hi(a, p, nc, L, s)) m2l_bcast_top(a, p, nc, L, s);
+    (void)(m2l_bcast_lo(a, p, nc, L, s) || m2l_bcast_hi(a, p, nc, L, s) || m2l_bcast_top(a, p, nc, L, s) ||
+           m2l_bcast_14(a, p, nc, L, s) || m2l_bcast_15(a, p, nc, L, s) || m2l_bcast_16(a, p, nc, L, s));
 }
 
 }  // namespace sfmm

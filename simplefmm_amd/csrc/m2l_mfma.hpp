@@ -10,8 +10,8 @@
 // target's local expansion is written once at the end (this kernel is the
 // first writer of L at every level >= 2).
 //
-// T = double: FP64 MFMA throughout.  T = float: FP32 MFMA stages with FP32
-// operands and FP64 accumulation across offsets (mixed precision).
+// FP32 MFMA stages with FP32 operands and FP64 accumulation across offsets: the
+// mixed path above p = 12 (FP64 runs m2l_bcast.hpp, mixed up to p = 12 m2l_dense.hpp).
 #pragma once
 
 #include <type_traits>
@@ -30,17 +30,6 @@ template <typename T>
 struct Mfma;
 
 template <>
-struct Mfma<double> {
-    typedef double V4 __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ V4 run(double a, double b, V4 c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    // row of D held in register r of lane l (16x16x4 f64 layout)
-    static __device__ __forceinline__ int drow(int lane, int r) { return 4 * r + (lane >> 4); }
-};
-
-template <>
 struct Mfma<float> {
     typedef float V4 __attribute__((ext_vector_type(4)));
     static __device__ __forceinline__ V4 run(float a, float b, V4 c)
@@ -48,8 +37,8 @@ struct Mfma<float> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
     // The FP32 operator fragments hold operator row 4 (i % 4) + i / 4 in MFMA
-    // row i, so the expansion row held in register r of lane l is 4 r + l / 16,
-    // as for FP64: register r covers rows [4r, 4r + 4) in both.
+    // row i, so the expansion row held in register r of lane l is 4 r + l / 16:
+    // register r covers rows [4r, 4r + 4).
     static __device__ __forceinline__ int drow(int lane, int r) { return 4 * r + (lane >> 4); }
 };
 
@@ -664,27 +653,18 @@ __device__ __forceinline__ void write_locals(const M2LArgs& a, int64_t blk, doub
 // i-2 and stage 3 on entry i-3; one barrier ends the phase.  Stage buffers
 // alternate by entry parity (G: stored columns, Y: after stage 1, Z: after
 // stage 2), so no two concurrent steps touch the same buffer.  Loads run ahead:
-// source columns kAhead<T> entries (with two, two register sets alternate by
-// phase parity), operators and the azimuth table one entry.  Entries outside [0, ne) run on
+// source columns kAhead<T> entries (two register sets alternate by phase
+// parity), operators and the azimuth table one entry.  Entries outside [0, ne) run on
 // zeroed or repeated data with zero azimuth factors, so they add nothing.
 constexpr int kCsSlots = 8;  // azimuth table slots in LDS, by entry index mod 8
 
-// Column prefetch distance: two entries for FP32 stages (which gather from
-// the FP32 copy of the multipoles), one for FP64 (a second set of FP64
-// columns would spill at p = 12).
+// Column prefetch distance in entries.
 template <typename T>
-constexpr int kAhead = sizeof(T) == 4 ? 2 : 1;
+constexpr int kAhead = 2;
 
-// Source expansions the kernel gathers from: M itself, or its FP32 copy.
+// Source expansions the kernel gathers from: the FP32 copy of the multipoles.
 template <typename T>
-__device__ __forceinline__ const T* m2l_source(const M2LArgs& a, const double* M);
-template <>
-__device__ __forceinline__ const double* m2l_source<double>(const M2LArgs&, const double* M)
-{
-    return M;
-}
-template <>
-__device__ __forceinline__ const float* m2l_source<float>(const M2LArgs& a, const double*)
+__device__ __forceinline__ const T* m2l_source(const M2LArgs& a, const double*)
 {
     return a.M32;
 }
@@ -818,15 +798,12 @@ __device__ __forceinline__ int64_t xcd_block(int64_t n_block)
     return static_cast<int64_t>(blockIdx.x % 8) * per + blockIdx.x / 8;
 }
 
-// Wavefronts per workgroup: 12 (3 per SIMD), measured best at p = 12 for both
-// stage precisions (FP32 against 8 and 16, FP64 against 8).  The sequential
-// kernel uses 8.
+// Wavefronts per workgroup: 12 (3 per SIMD), measured best against 8 and 16.
 template <typename T>
 __host__ __device__ constexpr int pipe_waves()
 {
     return 12;
 }
-constexpr int kSeqWaves = 8;
 
 template <typename T, int P, int NC>
 __global__ __launch_bounds__(64 * pipe_waves<T>(), 1) void m2l_pipe_kernel(M2LArgs a, const double* __restrict__ M,
@@ -862,117 +839,12 @@ __global__ __launch_bounds__(64 * pipe_waves<T>(), 1) void m2l_pipe_kernel(M2LAr
     }
 }
 
-// ---------------------------------------------------------------- sequential kernel
-// For orders whose six pipeline buffers exceed LDS (FP64, p > 12): one entry
-// at a time, four barriers per entry, loads issued one entry ahead.
-template <typename T, int P, int NC, int SC, int W>
-__device__ __forceinline__ void m2l_seq_wave(const M2LArgs& a, int64_t blk, int ne, const double* __restrict__ M,
-                                             double* __restrict__ L, T* Xs, T* Ys, T* cst, const int* ent_w,
-                                             const int* ent_s)
-{
-    using WS = WaveState<T, P, NC, SC, W>;
-    constexpr int TB = 16 / NC;
-    constexpr int NCS = 2 * (P + 1);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    Acc<WS::NJ, 1> acc;
-    acc.zero();
-    WS ws;
-    ws.init(tid);
-    const T* Msrc = m2l_source<T>(a, M);
-    Cols<WS::GI, T> cols;
-    ws.load_cols(cols, a, Msrc, ent_s);
-    double cs_next = 0.0;
-    if constexpr (W == 0) {
-        const double v = load_cs<P>(a, ent_w[0], lane);
-        cs_next = load_cs<P>(a, ent_w[ne > 1 ? 1 : 0], lane);
-        if (lane < NCS) cst[lane] = static_cast<T>(v);
-    }
-    {
-        const int w = ent_w[0];
-        const int cls = __builtin_amdgcn_readfirstlane(ent_class(w));
-        const int d2 = __builtin_amdgcn_readfirstlane(ent_dist(w));
-        ws.load_fwd(a, cls, lane);
-        ws.load_cx(a, d2, lane);
-        ws.load_back(a, cls, lane);
-    }
-    __syncthreads();
-    for (int e = 0; e < ne; ++e) {
-        // azimuth table: slot e & 1 holds entry e, slot (e + 1) & 1 receives entry e + 1
-        const T* cs = cst + (e & 1) * NCS;
-        ws.store_cols(Xs, cols, cs);
-        if constexpr (W == 0) {
-            cst[lane < NCS ? ((e + 1) & 1) * NCS + lane : 2 * NCS + lane] = static_cast<T>(cs_next);
-            cs_next = load_cs<P>(a, ent_w[e + 2 < ne ? e + 2 : ne - 1], lane);
-        }
-        ws.use_loaded();
-        const int en = e + 1 < ne ? e + 1 : e;  // the last entry reloads itself, harmlessly
-        ws.load_cols(cols, a, Msrc, ent_s + en * TB);
-        const int wn = ent_w[en], we = ent_w[e];
-        const int cn = __builtin_amdgcn_readfirstlane(ent_class(wn));
-        const int dn = __builtin_amdgcn_readfirstlane(ent_dist(wn));
-        const int c_e = __builtin_amdgcn_readfirstlane(ent_class(we));
-        const int d_e = __builtin_amdgcn_readfirstlane(ent_dist(we));
-        if (cn != c_e) {
-            ws.load_fwd(a, cn, lane);
-            ws.load_back(a, cn, lane);
-        }
-        if (dn != d_e) ws.load_cx(a, dn, lane);
-        __syncthreads();
-        StageIn<T, P, SC, W> in;
-        read_rot_fwd<T, P, SC, W>(in.b1, Xs, lane);
-        stage_rot_fwd<T, P, SC, W>(ws.a1, in.b1, Ys, lane);
-        __syncthreads();
-        read_coax<T, P, SC, W>(in.b2, Ys, lane);
-        stage_coax<T, P, SC, W>(ws.a2, in.b2, Xs, lane);
-        __syncthreads();
-        read_rot_back<T, P, SC, W>(in.b3, Xs, lane);
-        stage_rot_back<T, P, SC, W>(ws.a3, in.b3, cs, acc, lane);
-        __syncthreads();
-    }
-    write_locals<T, P, NC, SC, W>(a, blk, L, acc, lane);
-}
-
-template <typename T, int P, int NC>
-__global__ __launch_bounds__(64 * kSeqWaves, 1) void m2l_seq_kernel(M2LArgs a, const double* __restrict__ M,
-                                                                   double* __restrict__ L)
-{
-    constexpr int NTH = 64 * kSeqWaves;
-    constexpr int K = (P + 1) * (P + 1);
-    constexpr int TB = 16 / NC;
-    __shared__ T Xs[(K + kPadRows + 1) * kLdsW];
-    __shared__ T Ys[(K + kPadRows + 1) * kLdsW];
-    __shared__ alignas(16) T cst[4 * (P + 1) + 64];
-    __shared__ int ent_w[kMaxEntries];
-    __shared__ int ent_s[kMaxEntries * TB];
-    const int64_t blk = xcd_block(a.n_block);
-    if (blk >= a.n_block) return;
-    const int64_t e0 = a.blk_row[blk];
-    const int ne = static_cast<int>(a.blk_row[blk + 1] - e0);  // <= kMaxEntries (host-checked)
-    if (ne == 0) {
-        m2l_zero<P, NC>(a, blk, L);
-        return;
-    }
-    for (int i = threadIdx.x; i < kPadRows * kLdsW; i += NTH) {
-        Xs[K * kLdsW + i] = T(0);
-        Ys[K * kLdsW + i] = T(0);
-    }
-    for (int i = threadIdx.x; i < ne; i += NTH) ent_w[i] = a.ent_meta[e0 + i];
-    for (int i = threadIdx.x; i < ne * TB; i += NTH) ent_s[i] = a.ent_src[e0 * TB + i];
-    __syncthreads();
-    for_wave<0, kSeqWaves>(threadIdx.x >> 6, [&](auto wc) {
-        m2l_seq_wave<T, P, NC, 2 * kSeqWaves, decltype(wc)::value>(a, blk, ne, M, L, Xs, Ys, cst, ent_w, ent_s);
-    });
-}
-
 template <typename T, int P, int NC>
 void launch_one(const M2LArgs& a, const double* M, double* L, hipStream_t s)
 {
     const unsigned grid = static_cast<unsigned>(((a.n_block + 7) / 8) * 8);
-    if constexpr (pipe_fits<T, P, NC>())
-        hipLaunchKernelGGL((m2l_pipe_kernel<T, P, NC>), dim3(grid), dim3(64 * pipe_waves<T>()), 0, s, a, M, L);
-    else
-        hipLaunchKernelGGL((m2l_seq_kernel<T, P, NC>), dim3(grid), dim3(64 * kSeqWaves), 0, s, a, M, L);
+    static_assert(pipe_fits<T, P, NC>(), "the stage buffers exceed the LDS");
+    hipLaunchKernelGGL((m2l_pipe_kernel<T, P, NC>), dim3(grid), dim3(64 * pipe_waves<T>()), 0, s, a, M, L);
 }
 
 template <typename T, int P>
@@ -998,7 +870,6 @@ bool m2l_dispatch(const M2LArgs& a, int p, int nc, const double* M, double* L, h
 }
 
 // one translation unit per (type, order range) keeps the builds parallel
-bool m2l_f64_top(const M2LArgs& a, int p, int nc, const double* M, double* L, hipStream_t s);
 bool m2l_f32_top(const M2LArgs& a, int p, int nc, const double* M, double* L, hipStream_t s);
 
 }  // namespace sfmm

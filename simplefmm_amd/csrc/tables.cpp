@@ -218,11 +218,11 @@ void build_m2l_fragments(const Tables& t, bool interleave_rows, std::vector<doub
     }
 }
 
-void build_bcast_m2l(const Tables& t, std::vector<double>& rot, std::vector<double>& coax, std::vector<double>& az_fwd,
+void build_bcast_m2l(const Tables& t, int mode, std::vector<double>& rot, std::vector<double>& coax, std::vector<double>& az_fwd,
                      std::vector<double>& az_back)
 {
     const int P = t.p, NW = bcast_waves(P);
-    const BcastUnits ur = bcast_units(P, false), ut = bcast_units(P, true);
+    const BcastUnits ur = bcast_units(P, false, mode), ut = bcast_units(P, true, mode);
     const int rr = bcast_reg0(P, ur, false, NW), rt = bcast_reg0(P, ut, true, NW);
     rot.assign(static_cast<size_t>(70) * rr * 16, 0.0);
     coax.assign(static_cast<size_t>(28) * rt * 16, 0.0);

@@ -66,12 +66,12 @@ void build_m2l_fragments(const Tables& t, bool interleave_rows, std::vector<doub
 void build_dense_m2l(const Tables& t, std::vector<uint16_t>& ops, int& op_exp, std::vector<float>& az,
                      std::vector<int32_t>& off_grp);
 
-// Operators of the broadcast FP64 M2L (m2l_bcast.hpp, p <= kBcastMaxP): rot [70][registers][16]
+// Operators of the broadcast FP64 M2L (m2l_bcast.hpp) for the blocks of `mode` (BcastPart): rot [70][registers][16]
 // (forward; on coefficients whose order 0 is divided by sqrt 2 the back rotation is its
 // transpose), coax [28][registers][16], block elements column by column in the
 // wavefronts' order; az_fwd, az_back [343][16] pairs
 // (cos m phi - 1, sin m phi) and (cos m phi, sin m phi), m = 1..16 (0 above p).
-void build_bcast_m2l(const Tables& t, std::vector<double>& rot, std::vector<double>& coax, std::vector<double>& az_fwd,
+void build_bcast_m2l(const Tables& t, int mode, std::vector<double>& rot, std::vector<double>& coax, std::vector<double>& az_fwd,
                      std::vector<double>& az_back);
 
 // IEEE binary16 bits of x rounded to nearest even (|x| < 65520), and back.

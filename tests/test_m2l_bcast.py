@@ -28,7 +28,8 @@ int main()
 {
     for (int P = 1; P <= kBcastMaxP; ++P)
         for (int coax = 0; coax < 2; ++coax) {
-            const BcastUnits u = bcast_units(P, coax);
+          for (int mode = bcast_parted(P) ? 1 : 0; mode <= (bcast_parted(P) ? 2 : 0); ++mode) {
+            const BcastUnits u = bcast_units(P, coax, mode);
             int seen[20][2] = {}, most = 0, total = 0;
             for (int w = 0; w < bcast_waves(P); ++w) {
                 int cost = 0, last = -1;
@@ -46,9 +47,10 @@ int main()
             }
             for (int i = 0; i <= P; ++i)
                 for (int part = 0; part < 2; ++part)
-                    if (bcast_size(P, coax, i, part) > 0 && seen[i][part] != 1)
+                    if (seen[i][part] != (bcast_runs_part(mode, part) && bcast_size(P, coax, i, part) > 0))
                         return std::printf("FAIL block %d %d P=%d coax=%d: %d times\n", i, part, P, coax, seen[i][part]);
             if (most * bcast_waves(P) > 2 * total) return std::printf("FAIL balance P=%d coax=%d\n", P, coax);
+          }
         }
     std::printf("OK\n");
 }
@@ -121,7 +123,7 @@ TOLERANCE = 1e-13
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("p", range(1, 14))
+@pytest.mark.parametrize("p", range(1, 17))
 @pytest.mark.parametrize("gen,n,cap", [("uniform_cube", 2500, 40), ("sphere_shell", 6000, 16), ("uniform_cube", 40, 1)],
                          ids=["ragged", "sparse", "deep"])
 def test_matches_row_kernel(gen, n, cap, p):
