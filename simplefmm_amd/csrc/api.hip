@@ -1604,6 +1604,18 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
         P->dense_op_exp = dh->op_exp;
         P->dense_grp = dh->grp;
         P->dense_kd = sfmm::dense_order(p).kd;
+        // The dense M2L's default shape: a workgroup fills a compute unit and walks its
+        // block's offsets one after another, so while the blocks of 16 targets (4
+        // components) all run at once, 4 wavefronts on half the targets finish
+        // first (20k Plummer p = 12, ~200 blocks: 0.49 ms against 0.67 with 8); beyond, 8
+        // share each operator among twice the columns (4M uniform p = 10: 25.6 against 33.8).
+        int64_t blocks16 = 0;
+        for (int l = 2; l <= D; ++l) {
+            int64_t nodes[8] = {};
+            for (int32_t a = 0; a < t.lv[l].n_node(); ++a) ++nodes[t.lv[l].code[a] & 7];
+            for (int64_t c : nodes) blocks16 += (c + 15) / 16;
+        }
+        P->dense_waves = blocks16 <= 256 ? 4 : 8;
         const uint16_t* dops = nullptr;
         const float* dmax = nullptr;
         if ((rc = P->upload(ops, &dops)) || (rc = P->upload(az, &P->dense_az)) ||

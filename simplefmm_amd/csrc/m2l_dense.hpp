@@ -21,13 +21,22 @@
 //     x = H + L with H = f16(x), L = f16(x - H), and C += A_hi H + A_lo H +
 //     A_hi L runs on the f16 matrix cores with FP32 accumulation; D_c, scaled
 //     to the f16 range and split the same way, is copied into LDS by the LDS
-//     DMA one offset ahead (two buffers);
+//     DMA one offset ahead (two buffers), the sources' columns are requested one
+//     offset ahead into registers;
 //   * at the end of an azimuth group C is rotated back by e^{-i m phi} and
 //     added into the running FP32 sum S; each target's L~ is written once in
 //     FP64 at the end (the first writer of L at levels >= 2).  (Rotating the
 //     accumulators from group to group instead, without S, saves registers but
 //     rounds each earlier contribution once per later group: 3x the error.)
 // Orders 1..12 (the class operator of order 12 fills 66 KiB).
+//
+// 16M Plummer p = 12: 93.4 ms (98.2 before the columns came an offset ahead, the
+// splits moved between the products, and the loop's register copies, which waited
+// for every load in flight, went); 4M uniform p = 10: 25.6 (27.6).  Of an offset's
+// ~8,200 cycles the products take 99 x 16 x 2 per SIMD, and the 270 vector
+// instructions a wavefront runs beside them exceed the two per product that the
+// matrix cores hide (a third costs 5 cycles).  Left out to see: the operator copy
+// 14%, its fragments' LDS reads nothing, sources always in L2 5%, operators 2%.
 #pragma once
 
 #if !defined(__HIPCC__) && !defined(__host__)
@@ -248,12 +257,26 @@ __device__ __forceinline__ void dense_mma(const dh8& ahi, const dh8& alo, const 
     c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi, c, 0, 0, 0);
 }
 
+// Two tiles' products, alternating: each chain of three keeps its order.
+__device__ __forceinline__ void dense_mma2(const dh8* ahi, const dh8* alo, const dh8& bhi0, const dh8& blo0,
+                                           const dh8& bhi1, const dh8& blo1, df4& c0, df4& c1)
+{
+    c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[0], blo0, c0, 0, 0, 0);
+    c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[1], blo1, c1, 0, 0, 0);
+    c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[0], bhi0, c0, 0, 0, 0);
+    c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[1], bhi1, c1, 0, 0, 0);
+    c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[0], bhi0, c0, 0, 0, 0);
+    c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[1], bhi1, c1, 0, 0, 0);
+}
+
 // One 16-byte chunk per lane from global memory into LDS at dst + 16 * lane
 // (LDS DMA; dst is wave-uniform).
 __device__ __forceinline__ void dense_lds_copy(const dh8* src, dh8* dst)
 {
     __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
 }
+// Keeps the compiler from moving memory operations across this point.
+__device__ __forceinline__ void dense_fence() { asm volatile("" ::: "memory"); }
 // Waits until at most N vector memory loads of the wave are in flight (LDS DMA
 // included; they complete in issue order): with at least N loads issued after
 // an operator copy, the copy is done.
@@ -261,10 +284,12 @@ template <int N>
 __device__ __forceinline__ void dense_wait_loads()
 {
     static_assert(N >= 0 && N <= 63, "vmcnt range");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+    // the builtin, not assembly: the compiler then knows which loads have arrived
+    // and adds no wait of its own for them
+    dense_fence();
+    __builtin_amdgcn_s_waitcnt((N & 15) | 7 << 4 | 15 << 8 | (N >> 4) << 14);
+    dense_fence();
 }
-// Keeps the compiler from moving memory operations across this point.
-__device__ __forceinline__ void dense_fence() { asm volatile("" ::: "memory"); }
 
 // Fragment of tile t (cos tiles, then sin tiles) in K-step ks.
 template <int NKS>
@@ -330,9 +355,10 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
     const int64_t per = (a.n_block + 7) / 8;
     const int64_t blk = static_cast<int64_t>(blockIdx.x % 8) * per + blockIdx.x / 8;
     if (blk >= a.n_block) return;
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, q = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: so are the copy's and the buffers' offsets
     const int comp = w % NCW, grp = w / NCW;
-    const bool active = comp < NC;
+    const bool active = NCW == NC || comp < NC;
     const int ti = 16 * grp + (lane & 15);
     const int32_t tg = a.blk_tgt[blk * TB + ti];
     const int64_t e0 = a.blk_row[blk];
@@ -366,12 +392,12 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
     // a wave-uniform float held in a scalar register
     auto uniform = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
 
-    // copies the operator of class cls into an LDS buffer: CH / NW chunks of 1 KiB
-    // per wavefront, a fixed count so that the wait below can count them
-    auto dma = [&](int cls, dh8* __restrict__ buf) {
+    // copies chunks [from, to) of this wavefront's CH / NW chunks of 1 KiB of the
+    // operator of class cls into an LDS buffer
+    auto dma = [&](int cls, dh8* __restrict__ buf, int lane, int from, int to) {
         const dh8* src = static_cast<const dh8*>(a.ops) + static_cast<int64_t>(cls) * CH * 64;
 #pragma unroll
-        for (int c = 0; c < CH / NW; ++c)
+        for (int c = from; c < to; ++c)
             dense_lds_copy(src + (w + NW * c) * 64 + lane, buf + (w + NW * c) * 64);
     };
     auto src_ptr = [&](int32_t s) -> const float* {
@@ -391,119 +417,165 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
     df4 cc[MTC], cs[MTS], sumc[MTC], sums[MTS];
     for (int i = 0; i < MTC; ++i) cc[i] = sumc[i] = df4{};
     for (int i = 0; i < MTS; ++i) cs[i] = sums[i] = df4{};
-    // the source columns of the next K-step, loaded one K-step ahead (lane group q
-    // holds K = 8 q + 0..7 of each 32-wide K-step, cos then sin)
-    df8 xr = df8{}, xi = df8{};
-    const float* csp = a.zero;  // this lane's source of the current entry
-    int32_t src1 = -1;          // and of the next one
+    // the source columns of every K-step (lane group q holds K = 8 q + 0..7 of each
+    // 32-wide K-step, cos then sin), requested one entry ahead: a K-step's
+    // registers take the next entry's columns as soon as they are split.  (One
+    // K-step ahead, the columns queued behind the operator copy.)
+    df8 xr[NKS], xi[NKS];
+    for (int ks = 0; ks < NKS; ++ks) xr[ks] = xi[ks] = df8{};
+    int32_t src1 = -1;  // this lane's source of the next entry
     if (ne > 0) {
-        dma(a.ent_meta[e0] & 0xff, opbuf0);
-        csp = src_ptr(a.ent_src[e0 * TB + ti]);
+        dma(a.ent_meta[e0] & 0xff, opbuf0, lane, 0, CH / NW);
+        const float* csp = src_ptr(a.ent_src[e0 * TB + ti]);
         src1 = a.ent_src[(e0 + (ne > 1 ? 1 : 0)) * TB + ti];
         if (ne < 2) src1 = -1;
-        xr = *reinterpret_cast<const df8*>(csp + 8 * q);
-        xi = *reinterpret_cast<const df8*>(csp + KC + 8 * q);
+        dense_for<0, NKS>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value;
+            xr[ks] = *reinterpret_cast<const df8*>(csp + 32 * ks + 8 * q);
+            xi[ks] = *reinterpret_cast<const df8*>(csp + 32 * ks + KC + 8 * q);
+        });
     }
     __syncthreads();  // saz, smeta, srow_*
     float csx[P + 1], csy[P + 1];  // cos, sin of m phi of the current azimuth group, times sc
-    int i = 0, g = ne > 0 ? (smeta[0] >> 8) & 0xff : -1;
-    while (i < ne) {
+    auto factors = [&](int g) {
         for (int m = 0; m <= P; ++m) {
             csx[m] = uniform(saz[(g * (P + 1) + m) * 2] * sc);
             csy[m] = uniform(saz[(g * (P + 1) + m) * 2 + 1] * sc);
         }
-        int gn = -1;  // group of the entry after this group's run
-        // one entry; even entries read opbuf0 and fill opbuf1, odd ones the reverse
-        // (two arrays, so the reads are seen not to alias the copy in flight)
-        auto entry = [&](const dh8* __restrict__ cur, dh8* __restrict__ nxt) {
-            const bool more = i + 1 < ne;
-            // the lane group, re-read each entry, so that the per-lane azimuth
-            // factors of the slots shared by orders m and 0 are selected where they
-            // are used instead of being held in registers across the loop (which
-            // spilled the running sums)
-            int qv = q;
-            asm volatile("" : "+v"(qv));
-            const int nmeta = more ? smeta[i + 1] : -1;
-            // the operator of entry i is in LDS and every wave is done with entry i - 1.
-            // After its copy (issued at the top of entry i - 1) an active wave issued a
-            // source index and 4 x 16 bytes of source columns per K-step (loads complete
-            // in order); an idle one issued nothing
-            if (i == 0 || !active) dense_wait_loads<0>();
-            else dense_wait_loads<4 * NKS>();
-            __syncthreads();
-            if (more) dma(nmeta & 0xff, nxt);
-            dense_fence();
-            const float* nsp = src_ptr(src1);
-            src1 = i + 2 < ne ? a.ent_src[(e0 + i + 2) * TB + ti] : -1;
-            if (active) {
-                // A fragments of the 11-ish tiles of each K-step, one step ahead (the
-                // fences keep the compiler from loading further ahead, which would
-                // take the registers of the accumulators); tile t of K-step ks is
-                // fragment t * NKS + ks (cos tiles, then sin tiles)
-                constexpr int NT = MTC + MTS;
-                dh8 ah = cur[ks0_frag<NKS>(0, 0) * 128 + lane], al = cur[ks0_frag<NKS>(0, 0) * 128 + 64 + lane];
-                dense_for<0, NKS>([&](auto kc) {
-                    constexpr int ks = decltype(kc)::value;
-                    // nothing of this K-step moves into the previous one's MFMAs: its
-                    // columns arrive during them
-                    __builtin_amdgcn_sched_barrier(0);
-                    // B fragments of this K-step: rotate by e^{i m phi}, scale, split
-                    dh8 bch, bcl, bsh, bsl;
-                    dense_for<0, 8>([&](auto jc) {
-                        constexpr int j = decltype(jc)::value;
-                        constexpr int s = 8 * ks + j;
-                        constexpr int m = dense_slot_m(Cfg::O, s), z = dense_slot_zero(Cfg::O, s);
-                        float cm = csx[m], sm = csy[m];
-                        if constexpr (z != 0 && m != 0) {  // lane groups whose element is of order 0
-                            const bool zq = (z >> qv) & 1;
-                            cm = zq ? sc : cm;
-                            sm = zq ? 0.0f : sm;
-                        }
-                        const float xrj = xr[j], xij = xi[j];
-                        _Float16 hh, ll;
-                        dense_split(xrj * cm - xij * sm, hh, ll, neg1);
-                        bch[j] = hh;
-                        bcl[j] = ll;
-                        dense_split(xrj * sm + xij * cm, hh, ll, neg1);
-                        bsh[j] = hh;
-                        bsl[j] = ll;
-                    });
-                    // the columns of the next K-step, of this entry or of the next one (zeros
-                    // after the last entry)
-                    {
-                        const float* np = ks + 1 < NKS ? csp + 32 * (ks + 1) : nsp;
-                        xr = *reinterpret_cast<const df8*>(np + 8 * q);
-                        xi = *reinterpret_cast<const df8*>(np + KC + 8 * q);
+    };
+    int i = 0, g = -1;
+    if (ne > 0) {
+        g = __builtin_amdgcn_readfirstlane((smeta[0] >> 8) & 0xff);
+        factors(g);
+    }
+    // one entry, returning the group of the next (-1: none); even entries read opbuf0 and fill opbuf1, odd ones the reverse
+    // (two arrays, so the reads are seen not to alias the copy in flight)
+    auto entry = [&](const dh8* __restrict__ cur, dh8* __restrict__ nxt) {
+        const bool more = i + 1 < ne;
+        // the lane and its group, re-read each entry, so that the addresses and the
+        // per-lane azimuth factors of the slots shared by orders m and 0 are formed
+        // where they are used instead of being held in registers across the loop
+        // (which spilled the running sums)
+        int qv = q, lv = lane;
+        asm volatile("" : "+v"(qv), "+v"(lv));
+        const int nmeta = __builtin_amdgcn_readfirstlane(smeta[more ? i + 1 : i]);
+        // the operator of entry i is in LDS, this entry's columns are in registers
+        // (requested during the previous entry), and every wave is done with entry
+        // i - 1.  One wait for all of it before the next copy is issued: behind a copy
+        // in flight the compiler waits for everything, the copy included
+        dense_wait_loads<0>();
+        // (a plain barrier: the previous entry's fragment reads were all consumed, and
+        // __syncthreads would also wait for the columns in flight)
+        dense_fence();
+        __builtin_amdgcn_s_barrier();
+        dense_fence();
+        // The next operator's copy is issued piece by piece between the tiles (all at
+        // once, the wavefronts queue for it before their first products: 1,700 cycles
+        // of an entry's 8,500).  After the last entry once more, unused: a branch
+        // would make the compiler wait for every load in flight.
+        const int ncls = nmeta & 0xff;
+        dma(ncls, nxt, lv, 0, CH / NW);
+        dense_fence();
+        const float* nsp = src_ptr(src1);
+        asm volatile("" ::"v"(nsp));  // src1 is used up before its register is loaded again
+        src1 = a.ent_src[(e0 + (i + 2 < ne ? i + 2 : ne - 1)) * TB + ti];
+        if (active) {
+            // A fragments of the 11-ish tiles of each K-step, in pairs of tiles whose
+            // chains of three products alternate, one pair ahead (the fences keep the
+            // compiler from loading further ahead, which would take the registers of
+            // the accumulators); tile t of K-step ks is fragment t * NKS + ks (cos
+            // tiles, then sin tiles)
+            constexpr int NT = MTC + MTS, NTP = (NT + 1) / 2;
+            dh8 ah[2], al[2];
+            auto fetch = [&](auto pc, auto kc, dh8* h, dh8* l) {
+                constexpr int t = 2 * decltype(pc)::value, ks = decltype(kc)::value;
+                h[0] = cur[ks0_frag<NKS>(t, ks) * 128 + lv];
+                l[0] = cur[ks0_frag<NKS>(t, ks) * 128 + 64 + lv];
+                if constexpr (t + 1 < NT) {
+                    h[1] = cur[ks0_frag<NKS>(t + 1, ks) * 128 + lv];
+                    l[1] = cur[ks0_frag<NKS>(t + 1, ks) * 128 + 64 + lv];
+                }
+            };
+            fetch(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, ah, al);
+            // B fragments of a K-step: the columns rotated by e^{i m phi}, scaled and split,
+            // slot by slot.  Those of K-step ks + 1 are made between the products of
+            // K-step ks (two sets), in the shadow of the matrix cores; before, all
+            // wavefronts split and then all multiplied.
+            dh8 bch[2], bcl[2], bsh[2], bsl[2];
+            auto split = [&](auto kc, auto jc) {
+                constexpr int ks = decltype(kc)::value, j = decltype(jc)::value, B = ks & 1;
+                constexpr int s = 8 * ks + j;
+                constexpr int m = dense_slot_m(Cfg::O, s), z = dense_slot_zero(Cfg::O, s);
+                float cm = csx[m], sm = csy[m];
+                if constexpr (z != 0 && m != 0) {  // lane groups whose element is of order 0
+                    const bool zq = (z >> qv) & 1;
+                    cm = zq ? sc : cm;
+                    sm = zq ? 0.0f : sm;
+                }
+                const float xrj = xr[ks][j], xij = xi[ks][j];
+                _Float16 hh, ll;
+                dense_split(__builtin_fmaf(xrj, cm, -(xij * sm)), hh, ll, neg1);
+                bch[B][j] = hh;
+                bcl[B][j] = ll;
+                dense_split(__builtin_fmaf(xrj, sm, xij * cm), hh, ll, neg1);
+                bsh[B][j] = hh;
+                bsl[B][j] = ll;
+            };
+            dense_for<0, 8>([&](auto jc) { split(std::integral_constant<int, 0>{}, jc); });
+            dense_for<0, NKS>([&](auto kc) {
+                constexpr int ks = decltype(kc)::value;
+                __builtin_amdgcn_sched_barrier(0);
+                // the next entry's columns of this K-step, whose columns are split
+                // already (zeros after the last entry)
+                xr[ks] = *reinterpret_cast<const df8*>(nsp + 32 * ks + 8 * qv);
+                xi[ks] = *reinterpret_cast<const df8*>(nsp + 32 * ks + KC + 8 * qv);
+                dense_for<0, NTP>([&](auto pc) {
+                    constexpr int pr = decltype(pc)::value, t = 2 * pr;
+                    constexpr int pn = (pr + 1) % NTP, kn = pr + 1 < NTP ? ks : ks + 1;
+                    dh8 nh[2], nl[2];
+                    dense_fence();
+                    if constexpr (kn < NKS)
+                        fetch(std::integral_constant<int, pn>{}, std::integral_constant<int, kn>{}, nh, nl);
+                    df4& c0 = t < MTC ? cc[t < MTC ? t : 0] : cs[t < MTC ? 0 : t - MTC];
+                    constexpr int B = ks & 1;
+                    const dh8& h0 = t < MTC ? bch[B] : bsh[B];
+                    const dh8& l0 = t < MTC ? bcl[B] : bsl[B];
+                    if constexpr (t + 1 < NT) {
+                        constexpr int u = t + 1;
+                        df4& c1 = u < MTC ? cc[u < MTC ? u : 0] : cs[u < MTC ? 0 : u - MTC];
+                        dense_mma2(ah, al, h0, l0, u < MTC ? bch[B] : bsh[B], u < MTC ? bcl[B] : bsl[B], c0, c1);
+                    } else {
+                        dense_mma(ah[0], al[0], h0, l0, c0);
                     }
-                    dense_for<0, NT>([&](auto tc) {
-                        constexpr int t = decltype(tc)::value;
-                        constexpr int tn = (t + 1) % NT, kn = t + 1 < NT ? ks : ks + 1;
-                        dh8 nh, nl;
-                        dense_fence();
-                        if constexpr (kn < NKS) {
-                            nh = cur[ks0_frag<NKS>(tn, kn) * 128 + lane];
-                            nl = cur[ks0_frag<NKS>(tn, kn) * 128 + 64 + lane];
-                        }
-                        if constexpr (t < MTC) dense_mma(ah, al, bch, bcl, cc[t]);
-                        else dense_mma(ah, al, bsh, bsl, cs[t - MTC]);
-                        if constexpr (kn < NKS) {
-                            ah = nh;
-                            al = nl;
-                        }
-                    });
+                    if constexpr (ks + 1 < NKS)
+                        dense_for<8 * pr / NTP, 8 * (pr + 1) / NTP>(
+                            [&](auto jc) { split(std::integral_constant<int, ks + 1>{}, jc); });
+                    if constexpr (kn < NKS) {
+                        ah[0] = nh[0], al[0] = nl[0];
+                        if constexpr (2 * pn + 1 < NT) ah[1] = nh[1], al[1] = nl[1];
+                    }
                 });
-            }
-            csp = nsp;
-            return more ? (nmeta >> 8) & 0xff : -1;
-        };
-        do {
-            gn = (i & 1) == 0 ? entry(opbuf0, opbuf1) : entry(opbuf1, opbuf0);
-            ++i;
-        } while (gn == g);
-        // the group's contribution, rotated back, into the running sums
+            });
+        }
+        return more ? (nmeta >> 8) & 0xff : -1;
+    };
+    // after an entry: at the end of its group, the contribution, rotated back, into
+    // the running sums.  Even and odd entries follow each other in the text: a
+    // choice between two calls merges their registers by copies, which wait for the
+    // loads in flight (700-1100 cycles an entry)
+    auto next_group = [&](int gn) {
+        ++i;
+        if (gn == g) return;
         if (active) dense_flush<MTC, MTS>(cc, cs, sumc, sums, saz + g * (P + 1) * 2, srow_m, q);
         g = gn;
+        if (g >= 0) factors(g);
+    };
+    while (g >= 0) {
+        next_group(entry(opbuf0, opbuf1));
+        if (g < 0) break;
+        next_group(entry(opbuf1, opbuf0));
     }
+    dense_wait_loads<0>();  // no copy into LDS outlives the workgroup
     // L~ of the block's targets (first writer at its level), unscaled, in FP64
     if (!active || tg < 0) return;
     const double un = ldexp(1.0, -a.op_exp - sexp);
