@@ -500,15 +500,13 @@ int cut_m2l_blocks(sfmm_plan_s* P, int TB, const std::vector<int>& order, const 
     return SFMM_OK;
 }
 
-// Blocks of the mixed-precision M2L on the f16 matrix cores: 32 targets per
-// wave group (4 / waves-per-group groups per block), offsets in (azimuth
-// group, polar class, id) order so that each azimuth group is one run.
+// Blocks of the mixed-precision M2L on the f16 matrix cores: 16/nc targets per
+// wavefront, offsets in (azimuth group, polar class, id) order so that each
+// azimuth group is one run.
 int build_dense_blocks(sfmm_plan_s* P, int nc)
 {
     if (P->dns[nc].blk_row) return SFMM_OK;
-    // targets per block: 16 per group of waves, one wave per component
-    const int ncw = nc == 3 ? 4 : nc;
-    const int TB = 16 * (P->dense_waves / ncw);
+    const int TB = P->dense_waves * (16 / nc);
     const auto& cls = P->tables.off_class;
     const auto& grp = P->dense_grp;
     std::vector<int> order;
@@ -1619,7 +1617,7 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
         const uint16_t* dops = nullptr;
         const float* dmax = nullptr;
         if ((rc = P->upload(ops, &dops)) || (rc = P->upload(az, &P->dense_az)) ||
-            (rc = P->upload(std::vector<float>(P->dense_kd, 0.0f), &P->dense_zero)) ||
+            (rc = P->upload(std::vector<float>(4 * static_cast<size_t>(P->dense_kd), 0.0f), &P->dense_zero)) ||
             (rc = P->upload(std::vector<float>(static_cast<size_t>(4) * nnode, 0.0f), &dmax)))
             return rc;
         P->dense_ops = dops;

@@ -82,9 +82,9 @@ struct DenseArgs {
     const void* ops = nullptr;          // per class: [fragment][hi 64 | lo 64] x 8 halves (f16)
     const float* az = nullptr;          // [azimuth group][p+1][2] cos, sin of m phi
     const float* nodemax = nullptr;     // [gnode][nc] largest |value| of each FP32 multipole component
-    const float* zero = nullptr;        // zeros: the columns of absent sources
+    const float* zero = nullptr;        // zeros of 4 components: the columns of absent sources
     int op_exp = 0;                     // the operators are stored scaled by 2^op_exp
-    int waves = 8;                      // wavefronts per workgroup (4 or 8): 16 targets per wavefront group
+    int waves = 8;                      // wavefronts per workgroup (4 or 8): 16/nc targets each
 };
 
 // FP64 M2L with broadcast operators (m2l_bcast.hpp): groups of four rows of 16/nc
@@ -166,7 +166,7 @@ void launch_m2l(const DevPlan& d, int nc, const double* M, double* L, hipStream_
 void launch_l2l(const DevPlan& d, LevelSpan children, int nc, double* L, hipStream_t s);
 void launch_l2p(const DevPlan& d, int nc, const double* L, double* out, hipStream_t s);
 void launch_m2l_mfma(const M2LArgs& a, int p, int nc, const double* M, double* L, hipStream_t s);
-// p <= 12; M32: the multipoles in FP32, [gnode][nc][dense_order(p).kd] (m2l_dense.hpp)
+// p <= 12; M32: the multipoles in FP32, F32LayoutOf<p> (m2l_dense.hpp)
 void launch_m2l_dense(const DenseArgs& a, int p, int nc, const float* M32, double* L, hipStream_t s);
 void launch_m2l_bcast(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
 // The multipoles of `count` nodes, [nc][(p+1)^2], in the broadcast M2L's order [pair][nc][Re, Im].

@@ -66,7 +66,8 @@ __global__ __launch_bounds__(64) void fp32_copy_kernel(const double* __restrict_
         if constexpr (ROW % 4 == 0) {  // four slots per lane, 16-byte stores
             float4* y4 = reinterpret_cast<float4*>(y);
             for (int i = lane; i < nc * ROW / 4; i += 64) {
-                const int c = (4 * i) / ROW, j = 4 * i - c * ROW;
+                constexpr bool alt = F32LayoutOf<P>::L.dense;  // components alternate
+                const int c = alt ? i % nc : (4 * i) / ROW, j = alt ? 4 * (i / nc) : 4 * i - c * ROW;
                 float v[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {

@@ -12,9 +12,9 @@
 // (m >= 1).  This kernel stores D_c densely (70 classes, level independent) and
 // applies it as one matrix product per interaction offset:
 //   * a workgroup (8 wavefronts, two per SIMD, or 4) takes a block of targets of one
-//     level and child octant (they share their 189 candidate offsets); wave w
-//     holds component w % NCW of a group of 16 targets as the 16 columns of
-//     16x16x32 f16 MFMA tiles;
+//     level and child octant (they share their 189 candidate offsets); a
+//     wave holds 16/nc of them, the nc components of a target side by side, as
+//     the 16 columns of 16x16x32 f16 MFMA tiles;
 //   * the offsets present in the block are walked grouped by azimuth: the
 //     sources' columns are rotated by e^{i m phi} in FP32 registers and scaled
 //     (the largest value over the wavefront's sources to below 2^15), split as
@@ -30,13 +30,18 @@
 //     rounds each earlier contribution once per later group: 3x the error.)
 // Orders 1..12 (the class operator of order 12 fills 66 KiB).
 //
-// 16M Plummer p = 12: 93.4 ms (98.2 before the columns came an offset ahead, the
-// splits moved between the products, and the loop's register copies, which waited
-// for every load in flight, went); 4M uniform p = 10: 25.6 (27.6).  Of an offset's
-// ~8,200 cycles the products take 99 x 16 x 2 per SIMD, and the 270 vector
-// instructions a wavefront runs beside them exceed the two per product that the
-// matrix cores hide (a third costs 5 cycles).  Left out to see: the operator copy
-// 14%, its fragments' LDS reads nothing, sources always in L2 5%, operators 2%.
+// 16M Plummer p = 12: 98.2 -> 88.6 ms; 4M uniform p = 10: 27.6 -> 22.4 ms, since
+//   * the columns come an offset ahead, the splits move between the products, and
+//     the loop's register copies, which waited for every load in flight, are gone
+//     (93.4 / 25.6);
+//   * the components of a target sit in neighbouring lanes, whose loads are 64
+//     contiguous bytes (one component to a wave, every lane of a load touched its
+//     own line: the vector L1's accesses took 80% of the kernel's cycles).
+// Of an offset's ~7,700 cycles the products take 99 x 16 x 2 per SIMD.  Left out to
+// see (before the second step): the products 8%, the splits 8%, the operator copy
+// 14%, its fragments' LDS reads nothing, sources always in L2 5%, operators 2%: what
+// bounds it is the chain of an offset's loads, splits, products and barrier, two
+// wavefronts deep on a SIMD.
 #pragma once
 
 #if !defined(__HIPCC__) && !defined(__host__)
@@ -182,9 +187,11 @@ __host__ __device__ constexpr int dense_slot_zero(const DenseOrder& o, int s)
     return b;
 }
 
-// Layout of the FP32 copy of the multipoles that P2M and M2M write beside M for
-// the mixed-precision M2L: per (node, component) `row` floats, the real-form
-// coefficient r at pos[r] (dense order for p <= 12, unpermuted above).
+// Layout of the FP32 copy of the multipoles that the mixed-precision M2L reads:
+// per component `row` floats, the real-form coefficient r at place pos[r] (dense
+// order for p <= 12, unpermuted above); for p <= 12 the components of a node
+// alternate every four places ([node][place / 4][component][4]), so that the
+// lanes of one target, its components, load 64 contiguous bytes (4 components).
 template <int P>
 struct F32Layout {
     static constexpr bool dense = P <= kDenseMaxP;
@@ -277,20 +284,15 @@ __device__ __forceinline__ void dense_lds_copy(const dh8* src, dh8* dst)
 }
 // Keeps the compiler from moving memory operations across this point.
 __device__ __forceinline__ void dense_fence() { asm volatile("" ::: "memory"); }
-// Waits until at most N vector memory loads of the wave are in flight (LDS DMA
-// included; they complete in issue order): with at least N loads issued after
-// an operator copy, the copy is done.
-template <int N>
-__device__ __forceinline__ void dense_wait_loads()
+// Waits for every load of the wave, from memory (LDS DMA included) and from LDS.
+// The builtin, not assembly: the compiler then knows that they have arrived and
+// adds no wait of its own for them.
+__device__ __forceinline__ void dense_wait_all()
 {
-    static_assert(N >= 0 && N <= 63, "vmcnt range");
-    // the builtin, not assembly: the compiler then knows which loads have arrived
-    // and adds no wait of its own for them
     dense_fence();
-    __builtin_amdgcn_s_waitcnt((N & 15) | 7 << 4 | 15 << 8 | (N >> 4) << 14);
+    __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt 0, lgkmcnt 0
     dense_fence();
 }
-
 // Fragment of tile t (cos tiles, then sin tiles) in K-step ks.
 template <int NKS>
 __host__ __device__ constexpr int ks0_frag(int t, int ks) { return t * NKS + ks; }
@@ -330,14 +332,13 @@ __device__ __forceinline__ void dense_flush(df4* cc, df4* cs, df4* sumc, df4* su
 }
 
 template <int P, int NC, int NW>
-__global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const float* __restrict__ M32,
+__global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, const float* __restrict__ M32,
                                                            double* __restrict__ L)
 {
     using Cfg = DenseCfg<P>;
     constexpr int K = (P + 1) * (P + 1);
-    constexpr int NCW = NC == 3 ? 4 : NC;  // waves per target group (NC = 3: the fourth only copies)
-    constexpr int G = NW / NCW;            // target groups per block
-    constexpr int TB = 16 * G;             // targets per block
+    constexpr int TW = 16 / NC;            // targets per wave
+    constexpr int TB = NW * TW;            // targets per block
     constexpr int CH = Cfg::O.chunks;      // LDS copy chunks of one class (64 x 16 bytes each)
     constexpr int NKS = Cfg::O.nks, MTC = Cfg::O.mtc, MTS = Cfg::O.mts, KC = Cfg::O.kc, KD = Cfg::O.kd;
     static_assert(MTS <= MTC && 16 * MTC <= kDenseMaxRows, "row tiles");
@@ -357,19 +358,19 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
     if (blk >= a.n_block) return;
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: so are the copy's and the buffers' offsets
-    const int comp = w % NCW, grp = w / NCW;
-    const bool active = NCW == NC || comp < NC;
-    const int ti = 16 * grp + (lane & 15);
-    const int32_t tg = a.blk_tgt[blk * TB + ti];
+    const int col = lane & 15, comp = col - (col / NC) * NC;
+    const bool used = col / NC < TW;  // 3 components: the last column is empty
+    const int ti = w * TW + (used ? col / NC : 0);
+    const int32_t tg = used ? a.blk_tgt[blk * TB + ti] : -1;
     const int64_t e0 = a.blk_row[blk];
     const int ne = static_cast<int>(a.blk_row[blk + 1] - e0);
 
-    // scale of this wavefront's columns (its component of 16 neighbouring
+    // scale of this wavefront's columns (the components of neighbouring
     // targets): the largest |value| over their sources maps below 2^15, so
     // rotated values stay below 2^15.5 < 65504 and keep 22 bits down to 2^-18
     // of the largest; one value per wavefront keeps the azimuth factors scalar
     float mx = 0.0f;
-    if (active && tg >= 0 && q == 0) {
+    if (tg >= 0 && q == 0) {
         for (int i0 = 0; i0 < ne; i0 += 8) {
             int32_t sn[8];
 #pragma unroll
@@ -401,8 +402,8 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
             dense_lds_copy(src + (w + NW * c) * 64 + lane, buf + (w + NW * c) * 64);
     };
     auto src_ptr = [&](int32_t s) -> const float* {
-        const float* real = M32 + (static_cast<int64_t>(s < 0 ? 0 : s) * NC + comp) * KD;
-        return (active && s >= 0) ? real : a.zero;
+        const float* real = M32 + static_cast<int64_t>(s < 0 ? 0 : s) * NC * KD + 4 * comp;
+        return (used && s >= 0) ? real : a.zero;
     };
     for (int k = tid; k < kAzGroups * (P + 1) * 2; k += 64 * NW) saz[k] = a.az[k];
     for (int k = tid; k < ne; k += 64 * NW) smeta[k] = a.ent_meta[e0 + k];
@@ -418,11 +419,19 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
     for (int i = 0; i < MTC; ++i) cc[i] = sumc[i] = df4{};
     for (int i = 0; i < MTS; ++i) cs[i] = sums[i] = df4{};
     // the source columns of every K-step (lane group q holds K = 8 q + 0..7 of each
-    // 32-wide K-step, cos then sin), requested one entry ahead: a K-step's
+    // 32-wide K-step, cos and sin), requested one entry ahead: a K-step's
     // registers take the next entry's columns as soon as they are split.  (One
     // K-step ahead, the columns queued behind the operator copy.)
     df8 xr[NKS], xi[NKS];
     for (int ks = 0; ks < NKS; ++ks) xr[ks] = xi[ks] = df8{};
+    auto load_step = [&](const float* p, auto kc, int q) {
+        constexpr int ks = decltype(kc)::value;
+        // places 32 ks + 8 q + 0..7, in two pieces of four, NC components apart
+        const df4* c = reinterpret_cast<const df4*>(p) + (8 * ks + 2 * q) * NC;
+        const df4* d = c + KC / 4 * NC;
+        xr[ks] = __builtin_shufflevector(c[0], c[NC], 0, 1, 2, 3, 4, 5, 6, 7);
+        xi[ks] = __builtin_shufflevector(d[0], d[NC], 0, 1, 2, 3, 4, 5, 6, 7);
+    };
     int32_t src1 = -1;  // this lane's source of the next entry
     if (ne > 0) {
         dma(a.ent_meta[e0] & 0xff, opbuf0, lane, 0, CH / NW);
@@ -430,9 +439,7 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
         src1 = a.ent_src[(e0 + (ne > 1 ? 1 : 0)) * TB + ti];
         if (ne < 2) src1 = -1;
         dense_for<0, NKS>([&](auto kc) {
-            constexpr int ks = decltype(kc)::value;
-            xr[ks] = *reinterpret_cast<const df8*>(csp + 32 * ks + 8 * q);
-            xi[ks] = *reinterpret_cast<const df8*>(csp + 32 * ks + KC + 8 * q);
+            load_step(csp, kc, q);
         });
     }
     __syncthreads();  // saz, smeta, srow_*
@@ -463,10 +470,7 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
         // (requested during the previous entry), and every wave is done with entry
         // i - 1.  One wait for all of it before the next copy is issued: behind a copy
         // in flight the compiler waits for everything, the copy included
-        dense_wait_loads<0>();
-        // (a plain barrier: the previous entry's fragment reads were all consumed, and
-        // __syncthreads would also wait for the columns in flight)
-        dense_fence();
+        dense_wait_all();
         __builtin_amdgcn_s_barrier();
         dense_fence();
         // The next operator's copy is issued piece by piece between the tiles (all at
@@ -479,7 +483,7 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
         const float* nsp = src_ptr(src1);
         asm volatile("" ::"v"(nsp));  // src1 is used up before its register is loaded again
         src1 = a.ent_src[(e0 + (i + 2 < ne ? i + 2 : ne - 1)) * TB + ti];
-        if (active) {
+        {
             // A fragments of the 11-ish tiles of each K-step, in pairs of tiles whose
             // chains of three products alternate, one pair ahead (the fences keep the
             // compiler from loading further ahead, which would take the registers of
@@ -527,8 +531,7 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
                 __builtin_amdgcn_sched_barrier(0);
                 // the next entry's columns of this K-step, whose columns are split
                 // already (zeros after the last entry)
-                xr[ks] = *reinterpret_cast<const df8*>(nsp + 32 * ks + 8 * qv);
-                xi[ks] = *reinterpret_cast<const df8*>(nsp + 32 * ks + KC + 8 * qv);
+                load_step(nsp, kc, qv);
                 dense_for<0, NTP>([&](auto pc) {
                     constexpr int pr = decltype(pc)::value, t = 2 * pr;
                     constexpr int pn = (pr + 1) % NTP, kn = pr + 1 < NTP ? ks : ks + 1;
@@ -566,7 +569,7 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
     auto next_group = [&](int gn) {
         ++i;
         if (gn == g) return;
-        if (active) dense_flush<MTC, MTS>(cc, cs, sumc, sums, saz + g * (P + 1) * 2, srow_m, q);
+        dense_flush<MTC, MTS>(cc, cs, sumc, sums, saz + g * (P + 1) * 2, srow_m, q);
         g = gn;
         if (g >= 0) factors(g);
     };
@@ -575,9 +578,9 @@ __global__ __launch_bounds__(64 * NW) void m2l_dense_kernel(DenseArgs a, const f
         if (g < 0) break;
         next_group(entry(opbuf1, opbuf0));
     }
-    dense_wait_loads<0>();  // no copy into LDS outlives the workgroup
+    dense_wait_all();  // no copy into LDS outlives the workgroup
     // L~ of the block's targets (first writer at its level), unscaled, in FP64
-    if (!active || tg < 0) return;
+    if (tg < 0) return;
     const double un = ldexp(1.0, -a.op_exp - sexp);
     double* Lt = L + (static_cast<int64_t>(tg) * NC + comp) * K;
     dense_for<0, MTC>([&](auto mc) {
@@ -608,7 +611,7 @@ void launch_m2l_dense_pw(const DenseArgs& a, int nc, const float* M32, double* L
 }
 
 // a.waves (4 or 8) wavefronts per workgroup: the tile shape, which fixes the
-// targets per block the work lists were cut for (16 per wavefront group).
+// targets per block the work lists were cut for (16/nc per wavefront).
 template <int P>
 void launch_m2l_dense_p(const DenseArgs& a, int nc, const float* M32, double* L, hipStream_t s)
 {
