@@ -320,8 +320,8 @@ __device__ __forceinline__ void dense_flush(df4* cc, df4* cs, df4* sumc, df4* su
             if constexpr (mt < MTS) {
                 const int m = rowm[16 * mt + 4 * q + r];
                 const float c = az[2 * m], sn = az[2 * m + 1], ls = cs[mt][r];
-                sumc[mt][r] += lc * c + ls * sn;
-                sums[mt][r] += ls * c - lc * sn;
+                sumc[mt][r] += __builtin_fmaf(lc, c, ls * sn);
+                sums[mt][r] += __builtin_fmaf(ls, c, -(lc * sn));
             } else {
                 sumc[mt][r] += lc;  // rows of order 0 (and padding)
             }
@@ -502,7 +502,8 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
             };
             fetch(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, ah, al);
             // B fragments of a K-step: the columns rotated by e^{i m phi}, scaled and split,
-            // slot by slot.  Those of K-step ks + 1 are made between the products of
+            // slot by slot (the fused products written out, here and in the flush: which
+            // of two products is fused would otherwise change with the code around).  Those of K-step ks + 1 are made between the products of
             // K-step ks (two sets), in the shadow of the matrix cores; before, all
             // wavefronts split and then all multiplied.
             dh8 bch[2], bcl[2], bsh[2], bsl[2];
@@ -521,7 +522,7 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
                 dense_split(__builtin_fmaf(xrj, cm, -(xij * sm)), hh, ll, neg1);
                 bch[B][j] = hh;
                 bcl[B][j] = ll;
-                dense_split(__builtin_fmaf(xrj, sm, xij * cm), hh, ll, neg1);
+                dense_split(__builtin_fmaf(xij, cm, xrj * sm), hh, ll, neg1);
                 bsh[B][j] = hh;
                 bsl[B][j] = ll;
             };
