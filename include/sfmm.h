@@ -153,8 +153,8 @@ int sfmm_synchronize(sfmm_plan plan);
  * [0] gather, [1] P2M, [2] M2M, [3] M2L, [4] L2L, [5] L2P, [6] P2P, [7] scatter, [8] total. */
 int sfmm_last_stage_ms(sfmm_plan plan, float ms[9]);
 
-/* Records the stage times of each of the next `count` evaluations in its own set of
- * HIP events on the plan's stream (instead of only the last one); count <= 0 stops. */
+/* Records the stage times of each of the next `count` evaluations in a set of its own
+ * (instead of only the last one's); count <= 0 stops. */
 int sfmm_record_stages(sfmm_plan plan, int count);
 /* Stage times (as sfmm_last_stage_ms, 9 per evaluation) of the evaluations recorded
  * since sfmm_record_stages; ms holds room for `capacity` evaluations. */

@@ -344,7 +344,7 @@ class FMM3D:
         return dict(zip(STAGES, [float(x) for x in ms]))
 
     def record_stages(self, count: int):
-        """Keeps per-stage HIP-event times for each of the next `count` evaluations."""
+        """Keeps the stage times of each of the next `count` evaluations."""
         _check(lib().sfmm_record_stages(self.h, int(count)))
 
     def recorded_stage_ms(self, capacity: int) -> list:

@@ -217,7 +217,14 @@ struct sfmm_plan_s {
     double* hQ = nullptr;  // device staging for host-array calls
     double* hU = nullptr;
     int64_t stage_q = 0, stage_u = 0;
-    hipEvent_t ev[9] = {};
+    // stage times (kernels.hpp): the device clock at the start of each stage and at
+    // the end, and which of them an evaluation wrote
+    struct Stamps {
+        uint64_t* t = nullptr;  // [9], device
+        unsigned written = 0;
+    };
+    Stamps own;
+    double ticks_per_ms = 1e5;
     bool timed = false;
     int m2l_kernel = 0;
     sfmm::P2PItems p2p;                // near-field work items
@@ -249,8 +256,10 @@ struct sfmm_plan_s {
     sfmm::SelfCorr self;                // self-list corrections (empty without a self generator)
     std::vector<int64_t> slist_row, slist_val;  // far self pairs per particle, original order (_slist)
     std::vector<int64_t> m2m_lvl[5], l2l_lvl[5];  // first block of each level (+ end)
-    hipEvent_t* last_ev = nullptr;   // event set of the last evaluation
-    std::vector<hipEvent_t> rec_ev;  // sets of 9 events, one set per recorded evaluation
+    Stamps last;                     // of the last evaluation
+    std::vector<Stamps> rec;         // one per recorded evaluation
+    uint64_t* rec_mem = nullptr;     // their memory
+    size_t rec_cap = 0;
     int rec_count = 0, rec_used = 0;
 
     ~sfmm_plan_s()
@@ -265,9 +274,8 @@ struct sfmm_plan_s {
         (void)hipFree(hQ);
         (void)hipFree(hU);
         (void)hipFree(p2p_partial);
-        for (auto& e : ev)
-            if (e) (void)hipEventDestroy(e);
-        for (auto& e : rec_ev) (void)hipEventDestroy(e);
+        (void)hipFree(own.t);
+        (void)hipFree(rec_mem);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -856,47 +864,49 @@ int run(sfmm_plan_s* P, int kind, int ncharge, const double* dQ, double* dU, int
     return run_on(P, mode, nc, qdim, dQ, dU, which, P->stream, true);
 }
 
-// The evaluation's launches on stream s; `timed` records the stage events
+// The evaluation's launches on stream s; `timed` notes the stage times
 // (off while a graph is being captured).
 int run_on(sfmm_plan_s* P, sfmm::Mode mode, int nc, int qdim, const double* dQ, double* dU, int which,
            hipStream_t s, bool timed)
 {
     const sfmm::DevPlan& d = P->d;
     const int depth = P->tree->t.depth;
-    hipEvent_t* ev = P->ev;
-    if (timed && P->rec_used < P->rec_count) ev = &P->rec_ev[9 * static_cast<size_t>(P->rec_used++)];
-#define REC(k) \
-    if (timed) HIP_TRY(hipEventRecord(ev[k], s))
-    REC(0);
-    sfmm::launch_gather_charges(d, qdim, dQ, P->qbuf, s);
-    sfmm::launch_fill(P->obuf, static_cast<int64_t>(nc) * d.n, 0.0, s);
-    REC(1);
+    sfmm_plan_s::Stamps* set = nullptr;
+    if (timed) set = P->rec_used < P->rec_count ? &P->rec[P->rec_used++] : &P->own;
+    if (set) set->written = 0;
+    auto stamp = [&](int stage) -> uint64_t* {  // where a launch notes the start of a stage
+        if (!set) return nullptr;
+        set->written |= 1u << stage;
+        return set->t + stage;
+    };
+    sfmm::launch_gather_charges(d, qdim, dQ, P->qbuf, nc, P->obuf, stamp(0), s);
     const bool far = (which & SFMM_FAR) && depth >= 2;  // fmm.hpp:816-820
+    if (far) stamp(1);  // where the gather notes its end
     // the mixed M2L reads an FP32 copy of the multipoles (levels >= 2), made in
     // one pass before it (P2M and M2M write only the FP64 multipoles)
     float* M32 = P->precision == SFMM_MIXED ? P->M32 : nullptr;
     if (far) sfmm::launch_p2m(d, mode, nc, P->qbuf, P->M, s);
-    REC(2);
-    const sfmm::TransArgs& m2m = P->m2m[nc];
-    if (far)
+    if (far && depth > 2) {
+        sfmm::launch_stamp(stamp(2), s);
         for (int l = depth - 1; l >= 2; --l) {
             if (P->m2l_kernel == 0)
-                sfmm::launch_translate(m2m, level_blocks(P->m2m_lvl[nc], l), P->p, nc, false, P->M, s);
+                sfmm::launch_translate(P->m2m[nc], level_blocks(P->m2m_lvl[nc], l), P->p, nc, false, P->M, s);
             else
                 sfmm::launch_m2m(d, {P->level_first[l], P->level_first[l + 1] - P->level_first[l]}, nc, P->M, s);
         }
-    REC(3);
+    }
     if (far) {
         if (M32) {
             // and, for the dense M2L, the range of every FP32 multipole, which scales the columns
             const int64_t f2 = P->level_first[2];
             const int row = P->dense ? P->dense_kd : P->K;
             sfmm::launch_fp32_copy(P->M + f2 * nc * P->K, P->level_first.back() - f2, nc, P->p, M32 + f2 * nc * row,
-                                   P->dense ? P->dense_nodemax + f2 * nc : nullptr, s);
+                                   P->dense ? P->dense_nodemax + f2 * nc : nullptr, stamp(3), s);
         }
         if (P->bcast) {
             const int64_t f2 = P->level_first[2], pr = 2 * sfmm::bcast_pairs(P->p);
-            sfmm::launch_pair_copy(P->M + f2 * nc * P->K, P->level_first.back() - f2, nc, P->p, P->Mx + f2 * nc * pr, s);
+            sfmm::launch_pair_copy(P->M + f2 * nc * P->K, P->level_first.back() - f2, nc, P->p, P->Mx + f2 * nc * pr, stamp(3),
+                                   s);
             sfmm::BcastArgs A = P->bcg[nc];
             A.Mx = P->Mx;
             sfmm::launch_m2l_bcast(A, P->p, nc, P->L, s);
@@ -907,36 +917,52 @@ int run_on(sfmm_plan_s* P, sfmm::Mode mode, int nc, int qdim, const double* dQ, 
             A.M32 = P->M32;
             sfmm::launch_m2l_mfma(A, P->p, nc, P->M, P->L, s);
         }
-        else sfmm::launch_m2l(d, nc, P->M, P->L, s);
+        else {
+            sfmm::launch_stamp(stamp(3), s);
+            sfmm::launch_m2l(d, nc, P->M, P->L, s);
+        }
     }
-    REC(4);
-    if (far)
+    if (far && depth > 2) {
+        sfmm::launch_stamp(stamp(4), s);
         for (int l = 3; l <= depth; ++l) {
             if (P->m2l_kernel == 0)
                 sfmm::launch_translate(P->l2l[nc], level_blocks(P->l2l_lvl[nc], l), P->p, nc, true, P->L, s);
             else
                 sfmm::launch_l2l(d, {P->level_first[l], P->level_first[l + 1] - P->level_first[l]}, nc, P->L, s);
         }
-    REC(5);
-    if (far) sfmm::launch_l2p(d, nc, P->L, P->obuf, s);
-    REC(6);
+    }
+    if (far) {
+        sfmm::launch_stamp(stamp(5), s);
+        sfmm::launch_l2p(d, nc, P->L, P->obuf, s);
+    }
     if (which & SFMM_NEAR) {
+        sfmm::launch_stamp(stamp(6), s);
         sfmm::launch_p2p(d, P->p2p, mode, nc, P->qbuf, P->obuf, P->p2p_partial, s, P->precision == SFMM_MIXED,
                          P->p2p_tpl);
         sfmm::launch_self_correction(d, P->self, mode, nc, (which & SFMM_SELF_LIST) != 0, P->qbuf, P->obuf, s);
     }
-    REC(7);
-    sfmm::launch_scatter_outputs(d, nc, P->obuf, dU, s);
-    REC(8);
-#undef REC
+    sfmm::launch_scatter_outputs(d, nc, P->obuf, dU, stamp(7), s);
     HIP_TRY(hipGetLastError());
-    if (timed) {
-        P->last_ev = ev;
+    if (set) {
+        set->written |= 1u << 8;
+        P->last = *set;
         P->timed = true;
     }
     return SFMM_OK;
 }
 
+// Waits for the plan's stream and reads the stage times (8 stages, total) of one evaluation.
+int read_stages(sfmm_plan_s* P, const sfmm_plan_s::Stamps& set, float* ms)
+{
+    int64_t t[9];
+    HIP_TRY(hipMemcpyAsync(t, set.t, sizeof t, hipMemcpyDeviceToHost, P->stream));
+    HIP_TRY(hipStreamSynchronize(P->stream));
+    for (int k = 7; k >= 0; --k)  // a stage without launches takes no time
+        if (!(set.written >> k & 1)) t[k] = t[k + 1];
+    for (int k = 0; k < 8; ++k) ms[k] = static_cast<float>(static_cast<double>(t[k + 1] - t[k]) / P->ticks_per_ms);
+    ms[8] = static_cast<float>(static_cast<double>(t[8] - t[0]) / P->ticks_per_ms);
+    return SFMM_OK;
+}
 
 constexpr int kBatchMaxStreams = 8;
 
@@ -1307,7 +1333,12 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
     P->m2l_kernel = desc->m2l_kernel;
     HIP_TRY(hipGetDevice(&P->device));
     HIP_TRY(hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking));
-    for (auto& e : P->ev) HIP_TRY(hipEventCreate(&e));
+    if (dev_malloc(&P->own.t, 9 * sizeof(uint64_t)) != hipSuccess) return fail(SFMM_ERR_ALLOC, "hipMalloc failed (stage times)");
+    {
+        int khz = 0;
+        if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, P->device) == hipSuccess && khz > 0)
+            P->ticks_per_ms = khz;
+    }
     const sfmm::Tree& t = tree->t;
     const int p = P->p, K = P->K;
     P->tables = *tables_for(p);
@@ -1783,11 +1814,7 @@ int sfmm_last_stage_ms(sfmm_plan plan, float ms[9])
     if (!plan || !ms) return fail(SFMM_ERR_ARG, "null argument");
     if (!plan->timed) return fail(SFMM_ERR_STATE, "no evaluation has run yet");
     HIP_TRY(hipSetDevice(plan->device));
-    const hipEvent_t* ev = plan->last_ev;
-    HIP_TRY(hipEventSynchronize(ev[8]));
-    for (int k = 0; k < 8; ++k) HIP_TRY(hipEventElapsedTime(&ms[k], ev[k], ev[k + 1]));
-    HIP_TRY(hipEventElapsedTime(&ms[8], ev[0], ev[8]));
-    return SFMM_OK;
+    return read_stages(plan, plan->last, ms);
 }
 
 int sfmm_record_stages(sfmm_plan plan, int count)
@@ -1795,13 +1822,19 @@ int sfmm_record_stages(sfmm_plan plan, int count)
     if (!plan) return fail(SFMM_ERR_ARG, "null argument");
     HIP_TRY(hipSetDevice(plan->device));
     HIP_TRY(hipStreamSynchronize(plan->stream));
-    const size_t need = 9 * static_cast<size_t>(std::max(count, 0));
-    if (need > plan->rec_ev.size()) plan->last_ev = plan->ev;  // the vector may reallocate
-    plan->rec_ev.reserve(need);
-    while (plan->rec_ev.size() < need) {
-        hipEvent_t e;
-        HIP_TRY(hipEventCreate(&e));
-        plan->rec_ev.push_back(e);
+    const size_t need = static_cast<size_t>(std::max(count, 0));
+    if (need > plan->rec_cap) {
+        // the last evaluation's times may lie in the memory that goes
+        if (plan->last.t != plan->own.t) plan->timed = false;
+        (void)hipFree(plan->rec_mem);
+        plan->rec_mem = nullptr;
+        plan->rec_cap = 0;
+        plan->rec.clear();
+        plan->rec_count = plan->rec_used = 0;
+        if (dev_malloc(&plan->rec_mem, need * 9 * sizeof(uint64_t)) != hipSuccess)
+            return fail(SFMM_ERR_ALLOC, "hipMalloc failed (stage times)");
+        plan->rec_cap = need;
+        for (size_t k = 0; k < need; ++k) plan->rec.push_back({plan->rec_mem + 9 * k, 0});
     }
     plan->rec_count = std::max(count, 0);
     plan->rec_used = 0;
@@ -1814,10 +1847,7 @@ int sfmm_recorded_stage_ms(sfmm_plan plan, float* ms, int capacity, int* recorde
     HIP_TRY(hipSetDevice(plan->device));
     const int nrec = std::min(plan->rec_used, capacity);
     for (int r = 0; r < nrec; ++r) {
-        hipEvent_t* ev = &plan->rec_ev[9 * static_cast<size_t>(r)];
-        HIP_TRY(hipEventSynchronize(ev[8]));
-        for (int k = 0; k < 8; ++k) HIP_TRY(hipEventElapsedTime(&ms[9 * r + k], ev[k], ev[k + 1]));
-        HIP_TRY(hipEventElapsedTime(&ms[9 * r + 8], ev[0], ev[8]));
+        if (int rc = read_stages(plan, plan->rec[static_cast<size_t>(r)], ms + 9 * r)) return rc;
     }
     *recorded = plan->rec_used;
     return SFMM_OK;
@@ -1856,7 +1886,7 @@ int sfmm_direct(sfmm_plan plan, int kind, int ncharge, const double* Q, int64_t 
     hipError_t e = hipMemcpyAsync(dQ, Q, sizeof(double) * qdim * n, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(dt, targets, sizeof(int64_t) * ntarget, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        sfmm::launch_gather_charges(plan->d, qdim, dQ, plan->qbuf, s);
+        sfmm::launch_gather_charges(plan->d, qdim, dQ, plan->qbuf, 0, nullptr, nullptr, s);
         sfmm::launch_direct(plan->d, mode, nc, plan->qbuf, ntarget, dt, dout, part, nsplit, s);
         e = hipGetLastError();
     }

@@ -34,25 +34,36 @@ inline int grid_for(int64_t n, int b) { return static_cast<int>((n + b - 1) / b)
 
 // ------------------------------------------------------------------ charges
 __global__ void gather_charges_kernel(int64_t n, int qdim, const int32_t* __restrict__ perm,
-                                      const double* __restrict__ Q, double* __restrict__ q)
+                                      const double* __restrict__ Q, double* __restrict__ q, int nout,
+                                      double* __restrict__ out, uint64_t* stamp)
 {
-    const int64_t s = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int64_t o = perm[s];
-    for (int c = 0; c < qdim; ++c) q[c * n + s] = Q[o * qdim + c];
+    stage_stamp(stamp);
+    const int64_t s0 = static_cast<int64_t>(blockIdx.x) * blockDim.x, s = s0 + threadIdx.x;
+    if (s < n) {
+        const int64_t o = perm[s];
+        for (int c = 0; c < qdim; ++c) q[c * n + s] = Q[o * qdim + c];
+    }
+    // the block's outputs, which are contiguous
+    const int64_t end = min(n, s0 + blockDim.x) * nout;
+    for (int64_t i = s0 * nout + threadIdx.x; i < end; i += blockDim.x) out[i] = 0.0;
+    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) stamp[1] = wall_clock64();
 }
+
+__global__ void stamp_kernel(uint64_t* stamp) { stage_stamp(stamp); }
 
 // The sorted outputs are interleaved, out[slot * nout + c], so each particle's
 // values are one contiguous read; the caller's array is walked in its own
 // order (coalesced read-modify-write) and the sorted side gathered through the
 // inverse permutation.
 __global__ void scatter_outputs_kernel(int64_t n, int nout, const int32_t* __restrict__ iperm,
-                                       const double* __restrict__ out, double* __restrict__ U)
+                                       const double* __restrict__ out, double* __restrict__ U, uint64_t* stamp)
 {
+    stage_stamp(stamp);
     const int64_t o = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (o >= n) return;
     const int64_t s = iperm[o];
     for (int c = 0; c < nout; ++c) U[o * nout + c] += out[s * nout + c];
+    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) stamp[1] = wall_clock64();
 }
 
 __global__ void fill_kernel(double* x, int64_t count, double v)
@@ -265,8 +276,9 @@ __global__ __launch_bounds__(64) void p2m_kernel(DevPlan d, int mode, int nc, co
 // M [node][nc][K] -> [node][pair (n, m)][nc][Re, Im] (m = 0: Re / sqrt 2, Im = 0),
 // plus one node of zeros after the last.
 __global__ __launch_bounds__(256) void pair_copy_kernel(const double* __restrict__ M, int64_t count, int nc, int np,
-                                                        int K, double2* __restrict__ Mx)
+                                                        int K, double2* __restrict__ Mx, uint64_t* stamp)
 {
+    stage_stamp(stamp);
     const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int per = np * nc;
     const int64_t node = i / per;
@@ -963,14 +975,22 @@ struct M2LRun {
 
 }  // namespace
 
-void launch_gather_charges(const DevPlan& d, int qdim, const double* Q, double* q, hipStream_t s)
+void launch_gather_charges(const DevPlan& d, int qdim, const double* Q, double* q, int nout, double* out, uint64_t* stamp,
+                           hipStream_t s)
 {
-    hipLaunchKernelGGL(gather_charges_kernel, dim3(grid_for(d.n, 256)), dim3(256), 0, s, d.n, qdim, d.perm, Q, q);
+    hipLaunchKernelGGL(gather_charges_kernel, dim3(grid_for(d.n, 256)), dim3(256), 0, s, d.n, qdim, d.perm, Q, q, out ? nout : 0,
+                       out, stamp);
 }
 
-void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, hipStream_t s)
+void launch_stamp(uint64_t* stamp, hipStream_t s)
 {
-    hipLaunchKernelGGL(scatter_outputs_kernel, dim3(grid_for(d.n, 256)), dim3(256), 0, s, d.n, nout, d.iperm, out, U);
+    if (stamp) hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(64), 0, s, stamp);
+}
+
+void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, uint64_t* stamp, hipStream_t s)
+{
+    hipLaunchKernelGGL(scatter_outputs_kernel, dim3(grid_for(d.n, 256)), dim3(256), 0, s, d.n, nout, d.iperm, out, U,
+                       stamp);
 }
 
 void launch_fill(double* x, int64_t count, double v, hipStream_t s)
@@ -985,12 +1005,12 @@ void launch_p2m(const DevPlan& d, Mode mode, int nc, const double* q, double* M,
     with_p<P2MRun>(d.p, d, static_cast<int>(mode), ncq, nc, q, M, s);
 }
 
-void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx, hipStream_t s)
+void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx, uint64_t* stamp, hipStream_t s)
 {
     const int np = (p + 1) * (p + 2) / 2;
     const int64_t total = (count + 1) * np * nc;
     hipLaunchKernelGGL(pair_copy_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s, M, count, nc,
-                       np, (p + 1) * (p + 1), reinterpret_cast<double2*>(Mx));
+                       np, (p + 1) * (p + 1), reinterpret_cast<double2*>(Mx), stamp);
 }
 
 void launch_l2p(const DevPlan& d, int nc, const double* L, double* out, hipStream_t s)

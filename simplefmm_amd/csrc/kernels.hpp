@@ -15,6 +15,17 @@ enum Mode : int {
     MODE_POTGRAD = 2,  // scalar charge -> potential and its gradient (4 outputs)
 };
 
+// Stage times are device clocks that light kernels write as they run, and a launch
+// of its own (launch_stamp) where a stage begins with a heavy one: a store or another
+// branch ahead of the work of P2M, L2P or P2P costs them scalar loads and registers
+// (L2P at p = 16: 95 us, and 120 with it).  Events between the stages held the stream
+// up instead: a 2k evaluation took 75 us with them and takes 37, one of 5k 447 and
+// 405, 20k mixed 387 and 375; no difference from 100k on.  Null: not noted.
+__device__ __forceinline__ void stage_stamp(uint64_t* p)
+{
+    if (p && (blockIdx.x | threadIdx.x) == 0) *p = wall_clock64();
+}
+
 // Device view of everything a launch needs.  All pointers are device memory.
 struct DevPlan {
     int p = 0, K = 0, depth = 0;
@@ -158,8 +169,12 @@ struct TransArgs {
 constexpr int64_t kTrSplitBlocks = 192;
 
 // All launches are asynchronous on `stream`.
-void launch_gather_charges(const DevPlan& d, int qdim, const double* Q, double* q, hipStream_t s);
-void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, hipStream_t s);
+// Charges to sorted order, and the sorted outputs (nout per particle; out null: none)
+// cleared.  Notes its start at stamp[0] and its end at stamp[1].
+void launch_gather_charges(const DevPlan& d, int qdim, const double* Q, double* q, int nout, double* out, uint64_t* stamp,
+                           hipStream_t s);
+void launch_stamp(uint64_t* stamp, hipStream_t s);
+void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, uint64_t* stamp, hipStream_t s);
 void launch_p2m(const DevPlan& d, Mode mode, int nc, const double* q, double* M, hipStream_t s);
 void launch_m2m(const DevPlan& d, LevelSpan parents, int nc, double* M, hipStream_t s);
 void launch_m2l(const DevPlan& d, int nc, const double* M, double* L, hipStream_t s);
@@ -170,11 +185,12 @@ void launch_m2l_mfma(const M2LArgs& a, int p, int nc, const double* M, double* L
 void launch_m2l_dense(const DenseArgs& a, int p, int nc, const float* M32, double* L, hipStream_t s);
 void launch_m2l_bcast(const BcastArgs& a, int p, int nc, double* L, hipStream_t s);
 // The multipoles of `count` nodes, [nc][(p+1)^2], in the broadcast M2L's order [pair][nc][Re, Im].
-void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx, hipStream_t s);
+void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx, uint64_t* stamp, hipStream_t s);
 // The FP32 copy (F32LayoutOf<p>: the dense M2L's layout for p <= 12, else the
 // real-form order) of `count` nodes of nc x (p+1)^2 FP64 coefficients, with
 // their per-component largest |value| into nodemax when it is not null.
-void launch_fp32_copy(const double* M, int64_t count, int nc, int p, float* M32, float* nodemax, hipStream_t s);
+void launch_fp32_copy(const double* M, int64_t count, int nc, int p, float* M32, float* nodemax, uint64_t* stamp,
+                      hipStream_t s);
 // upper = false: M2M (parents written); true: L2L (children added to).
 void launch_translate(const TransArgs& a, LevelSpan blocks, int p, int nc, bool upper, double* io, hipStream_t s);
 int translate_nfrag(int p, bool upper);

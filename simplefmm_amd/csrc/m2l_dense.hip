@@ -39,8 +39,9 @@ struct F32RowsOf {
 // when nodemax is given, the largest |value| per component is kept.
 template <int P>
 __global__ __launch_bounds__(64) void fp32_copy_kernel(const double* __restrict__ M, int64_t count, int nc,
-                                                       float* __restrict__ M32, float* __restrict__ nodemax)
+                                                       float* __restrict__ M32, float* __restrict__ nodemax, uint64_t* stamp)
 {
+    stage_stamp(stamp);
     constexpr int K = (P + 1) * (P + 1);
     constexpr int ROW = F32LayoutOf<P>::L.row;
     __shared__ double xs[4 * K];
@@ -97,23 +98,26 @@ __global__ __launch_bounds__(64) void fp32_copy_kernel(const double* __restrict_
 }
 
 template <int P>
-bool fp32_copy_p(int p, const double* M, int64_t count, int nc, float* M32, float* nodemax, hipStream_t s)
+bool fp32_copy_p(int p, const double* M, int64_t count, int nc, float* M32, float* nodemax, uint64_t* stamp,
+                 hipStream_t s)
 {
     if constexpr (P > 16) {
         return false;
     } else {
-        if (p != P) return fp32_copy_p<P + 1>(p, M, count, nc, M32, nodemax, s);
+        if (p != P) return fp32_copy_p<P + 1>(p, M, count, nc, M32, nodemax, stamp, s);
         const unsigned grid = static_cast<unsigned>(std::min<int64_t>(32768, count));
-        hipLaunchKernelGGL(fp32_copy_kernel<P>, dim3(grid), dim3(64), 0, s, M, count, nc, M32, nodemax);
+        hipLaunchKernelGGL(fp32_copy_kernel<P>, dim3(grid), dim3(64), 0, s, M, count, nc, M32, nodemax,
+                           stamp);
         return true;
     }
 }
 
 }  // namespace
 
-void launch_fp32_copy(const double* M, int64_t count, int nc, int p, float* M32, float* nodemax, hipStream_t s)
+void launch_fp32_copy(const double* M, int64_t count, int nc, int p, float* M32, float* nodemax, uint64_t* stamp,
+                      hipStream_t s)
 {
-    if (count > 0) (void)fp32_copy_p<1>(p, M, count, nc, M32, nodemax, s);
+    if (count > 0) (void)fp32_copy_p<1>(p, M, count, nc, M32, nodemax, stamp, s);
 }
 
 }  // namespace sfmm

@@ -171,3 +171,26 @@ def test_shifts_of_levels_around_the_split(cells, p):
         out.append(U)
     # the same sums in another order: a few thousand terms, 1.1e-16 each
     assert rel_l2(out[0], out[1]) < 1e-13
+
+
+@pytest.mark.parametrize("m2l_kernel,prec", [(0, api.FP64), (1, api.FP64), (0, api.MIXED)])
+def test_stage_times_of_evaluations_with_and_without_a_far_field(m2l_kernel, prec):
+    pos = np.random.default_rng(3).uniform(size=(20000, 3))
+    part = api.OctreePartitioner(pos, api.Box(corner=[0.0, 0.0, 0.0], width=1.0)).refine(8, 40)
+    fmm = api.FMM3D(part, 6, ncharge=1, m2l_kernel=m2l_kernel, precision=prec)
+    q, U = np.ones(len(pos)), np.zeros((len(pos), 4))
+    kinds = [api.BOTH, api.NEAR, api.FAR]
+    fmm.record_stages(len(kinds))
+    for which in kinds:
+        fmm.rinv_potgrad(q, U, which)
+    sets = fmm.recorded_stage_ms(8)
+    assert len(sets) == len(kinds)
+    fmm.record_stages(0)
+    fmm.rinv_potgrad(q, U)
+    for which, s in zip(kinds + [api.BOTH], sets + [fmm.stage_ms()]):
+        print(which, s, flush=True)
+        *stages, total = s.values()
+        absent = [[], [1, 2, 3, 4, 5], [6]][kinds.index(which)]
+        assert all((t == 0.0) == (k in absent) and t >= 0.0 for k, t in enumerate(stages))
+        # each is a difference of clocks, rounded to single precision
+        assert total == pytest.approx(sum(stages), rel=1e-5) and total < 1e3
