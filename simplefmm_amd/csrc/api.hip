@@ -810,8 +810,10 @@ int build_translate_blocks(sfmm_plan_s* P, int nc)
         return rc;
     // M2M partial sums of the levels that run split
     int64_t most = 0;
-    for (int l = 2; l < t.depth; ++l)
-        if (lv_m[l + 1] - lv_m[l] <= sfmm::kTrSplitBlocks) most = std::max(most, lv_m[l + 1] - lv_m[l]);
+    for (int l = 2; l < t.depth; ++l) {
+        const int64_t blocks = lv_m[l + 1] - lv_m[l];
+        if (blocks <= sfmm::tr_split_most(P->p, false)) most = std::max(most, std::min(blocks, sfmm::kTrSplitChunk));
+    }
     if (most > 0) {
         void* part = nullptr;
         if (dev_malloc(&part, sizeof(double) * static_cast<size_t>(most) * 8 * P->K * 16) != hipSuccess)

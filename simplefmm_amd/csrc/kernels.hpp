@@ -161,12 +161,21 @@ struct TransArgs {
     const int32_t* ent_oct = nullptr;   // child octant per entry
     const int32_t* ent_node = nullptr;  // [entries][16/nc] child gnodes, -1 = none
     const double* frag = nullptr;      // [8][nfrag][64]
-    // M2M partial sums of levels of at most kTrSplitBlocks blocks, [block][8][(p+1)^2][16]
+    // M2M partial sums of a split level, [block < kTrSplitChunk][8][(p+1)^2][16]
     double* part = nullptr;
 };
 // Levels of at most this many blocks run one workgroup per entry instead of one
-// per block: below it the blocks leave compute units idle.
-constexpr int64_t kTrSplitBlocks = 192;
+// per block.  M2M: below it the blocks leave compute units idle, above it the
+// partial sums cost more than that (whole / split, us: 291 blocks at p = 12 57 / 55,
+// 1142 135 / 211; 794 at p = 4 15 / 23).  L2L has no partial sums (291 blocks 79 / 54,
+// 1142 198 / 190, 1403 236 / 231 at p = 12; 794 at p = 4 17 / 19, p = 8 63 / 59).  At
+// p = 16 a wavefront of a whole block would need 280 registers and run alone on its
+// SIMD (1403 blocks: M2M 2115 / 943, L2L 1800 / 578): all levels, M2M in chunks.
+constexpr int64_t kTrSplitChunk = 1024;
+constexpr int64_t tr_split_most(int p, bool upper)
+{
+    return p >= 16 ? INT64_MAX : upper && p >= 8 ? 1024 : 192;
+}
 
 // All launches are asynchronous on `stream`.
 // Charges to sorted order, and the sorted outputs (nout per particle; out null: none)

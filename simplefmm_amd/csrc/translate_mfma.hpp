@@ -9,6 +9,7 @@
 //        the parents once.
 //   L2L: it gathers the parents into LDS once; for every entry it multiplies
 //        them by the octant's operator and adds the result to the children.
+// Small levels spread a block's entries over workgroups (translate_split_kernel).
 #pragma once
 
 #include <type_traits>
@@ -275,8 +276,8 @@ __global__ __launch_bounds__(64 * kTrWaves) void translate_kernel(TransArgs a, i
     });
 }
 
-// Small levels: a workgroup per entry (grid y: the block's entries), so that a
-// level takes one entry's time instead of up to eight in a row.  L2L entries
+// Small levels (tr_split_most): a workgroup per entry (grid y: the block's entries), so
+// that a level takes one entry's time instead of up to eight in a row.  L2L entries
 // write different children.  M2M entries of a block write partial sums, which
 // translate_sum_kernel adds in entry order (a second launch: handing them to the
 // block's last workgroup takes device-scope fences, 200 us at 128 blocks).
@@ -323,20 +324,27 @@ __global__ __launch_bounds__(256) void translate_sum_kernel(TransArgs a, int nc,
 template <int P, bool UPPER>
 void translate_nc(const TransArgs& a, LevelSpan b, int nc, double* io, hipStream_t s)
 {
-    if (b.count <= kTrSplitBlocks) {
-        hipLaunchKernelGGL((translate_split_kernel<P, UPPER>), dim3(static_cast<unsigned>(b.count), 8),
-                           dim3(64 * kTrSplitWaves), 0, s, a, nc, b.first, io);
-        if constexpr (!UPPER)
-            hipLaunchKernelGGL((translate_sum_kernel<P>), dim3(static_cast<unsigned>((b.count * tr_K(P) * 16 + 255) / 256)),
-                               dim3(256), 0, s, a, nc, b.first, b.count, io);
+    constexpr int64_t most = tr_split_most(P, UPPER);
+    if (b.count <= most) {
+        const int64_t chunk = UPPER ? b.count : kTrSplitChunk;
+        for (int64_t at = 0; at < b.count; at += chunk) {
+            const int64_t first = b.first + at, count = b.count - at < chunk ? b.count - at : chunk;
+            hipLaunchKernelGGL((translate_split_kernel<P, UPPER>), dim3(static_cast<unsigned>(count), 8),
+                               dim3(64 * kTrSplitWaves), 0, s, a, nc, first, io);
+            if constexpr (!UPPER)
+                hipLaunchKernelGGL((translate_sum_kernel<P>), dim3(static_cast<unsigned>((count * tr_K(P) * 16 + 255) / 256)),
+                                   dim3(256), 0, s, a, nc, first, count, io);
+        }
         return;
     }
-    const dim3 grid(static_cast<unsigned>(b.count)), blk(64 * kTrWaves);
-    switch (nc) {
-    case 1: hipLaunchKernelGGL((translate_kernel<P, 1, UPPER>), grid, blk, 0, s, a, b.first, io); break;
-    case 2: hipLaunchKernelGGL((translate_kernel<P, 2, UPPER>), grid, blk, 0, s, a, b.first, io); break;
-    case 3: hipLaunchKernelGGL((translate_kernel<P, 3, UPPER>), grid, blk, 0, s, a, b.first, io); break;
-    default: hipLaunchKernelGGL((translate_kernel<P, 4, UPPER>), grid, blk, 0, s, a, b.first, io); break;
+    if constexpr (most < INT64_MAX) {
+        const dim3 grid(static_cast<unsigned>(b.count)), blk(64 * kTrWaves);
+        switch (nc) {
+        case 1: hipLaunchKernelGGL((translate_kernel<P, 1, UPPER>), grid, blk, 0, s, a, b.first, io); break;
+        case 2: hipLaunchKernelGGL((translate_kernel<P, 2, UPPER>), grid, blk, 0, s, a, b.first, io); break;
+        case 3: hipLaunchKernelGGL((translate_kernel<P, 3, UPPER>), grid, blk, 0, s, a, b.first, io); break;
+        default: hipLaunchKernelGGL((translate_kernel<P, 4, UPPER>), grid, blk, 0, s, a, b.first, io); break;
+        }
     }
 }
 

@@ -173,6 +173,26 @@ def test_shifts_of_levels_around_the_split(cells, p):
     assert rel_l2(out[0], out[1]) < 1e-13
 
 
+@pytest.mark.parametrize("cells,p", [(4096, 8), (4097, 8), (4096, 16), (4097, 16)])
+def test_shifts_of_a_level_around_1024_blocks(cells, p):
+    # 4 parents to a block of 4 components: the L2L's change from p = 8 on, and at
+    # p = 16 the M2M's chunk
+    rng = np.random.default_rng(cells)
+    at = rng.permutation(32**3)[:cells]
+    corner = np.stack([at // 1024, at // 32 % 32, at % 32], 1)
+    pos = ((corner[:, None, :] + rng.uniform(size=(cells, 5, 3))) / 32).reshape(-1, 3)
+    part = api.OctreePartitioner(pos, api.Box(corner=[0.0, 0.0, 0.0], width=1.0)).refine(20, 4)
+    q = rng.uniform(-1, 1, len(pos))
+    out = []
+    for kernel in (0, 1):
+        print(f"cells={cells} p={p} m2l_kernel={kernel} depth={part.level()}", flush=True)
+        U = np.zeros((len(pos), 4))
+        api.FMM3D(part, p, ncharge=1, m2l_kernel=kernel).rinv_potgrad(q, U, api.FAR)
+        out.append(U)
+    # the same sums in another order: a few thousand terms, 1.1e-16 each
+    assert rel_l2(out[0], out[1]) < 1e-13
+
+
 @pytest.mark.parametrize("m2l_kernel,prec", [(0, api.FP64), (1, api.FP64), (0, api.MIXED)])
 def test_stage_times_of_evaluations_with_and_without_a_far_field(m2l_kernel, prec):
     pos = np.random.default_rng(3).uniform(size=(20000, 3))
