@@ -318,7 +318,7 @@ def main() -> int:
             split = p <= 12
             peak, kernel = (PEAK_F16, "m2l_dense_kernel (f16 split)") if split else (PEAK_FP32, "m2l_pipe_kernel (fp32)")
         else:
-            peak, kernel = PEAK_FP64, "m2l_pipe_kernel (fp64)"
+            peak, kernel = PEAK_FP64, "m2l_bcast_kernel (fp64)"
             split = False
         # algorithmic flops: the complex full-m count of rotate-translate-rotate per
         # (pair, component); executed: what the kernel's arithmetic needs without padding

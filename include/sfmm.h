@@ -104,14 +104,14 @@ int sfmm_tree_level_lists(sfmm_tree tree, int level, int64_t* c_node, int64_t* l
 
 typedef struct {
     int p;                    /* expansion order, 1..16 (FMM3D template p)            */
-    int precision;            /* SFMM_FP64 or SFMM_MIXED (FP32 MFMA M2L stages, FP64 accumulation) */
+    int precision;            /* SFMM_FP64 or SFMM_MIXED (M2L in split f16 or FP32 on the matrix cores, FP32 near pairs) */
     int max_ncharge;          /* largest ncharge later passed to SFMM_POTENTIAL (1..4) */
     /* optional self lists (FMM3D(partitioner, comm, self_generator), fmm.hpp:204):
      * self_generator(i) = self_val[self_row[i] .. self_row[i+1]) (original indices,
      * self_row[0] = 0); NULL means self_generator(i) = {i}.  Copied at creation. */
     const int64_t* self_row;
     const int64_t* self_val;
-    int m2l_kernel;           /* 0: offset-grouped MFMA (default); 1: row-parallel VALU kernel */
+    int m2l_kernel;           /* 0: offset-grouped (default); 1: one workgroup per target row by row */
 } sfmm_plan_desc;
 
 /* FMM3D(partitioner, comm[, self_generator]): fmm.hpp:204-427.  Uploads the tree

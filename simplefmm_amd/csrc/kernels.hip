@@ -632,7 +632,7 @@ __device__ __forceinline__ void pair_kernel_f32(float dx, float dy, float dz, co
 }
 
 // Near field (N2N, fmm.hpp:773-809), one wavefront per work item.  An item is
-// a target leaf and a run of at most a few thousand sources of its near list
+// a target leaf and a run of its near list, at most a limit of pairs for the tree
 // (the concatenation of its merged source ranges): leaves whose near list is
 // long (coarse leaves next to deep subtrees) are split over several items so
 // that no wavefront carries a long tail.  Each lane holds T targets (T = 1, 2
