@@ -279,23 +279,24 @@ __global__ __launch_bounds__(256) void pair_copy_kernel(const double* __restrict
                                                         int K, double2* __restrict__ Mx, uint64_t* stamp)
 {
     stage_stamp(stamp);
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int per = np * nc;
-    const int64_t node = i / per;
-    if (node > count) return;
-    const int k = static_cast<int>(i - node * per);
-    const int pr = k / nc, c = k - pr * nc;
-    int n = static_cast<int>((sqrtf(8.0f * pr + 1.0f) - 1.0f) * 0.5f);
-    while ((n + 1) * (n + 2) / 2 <= pr) ++n;
-    while (n * (n + 1) / 2 > pr) --n;
-    const int m = pr - n * (n + 1) / 2;
-    double2 v{0.0, 0.0};
-    if (node < count) {
-        const double* Mn = M + (node * nc + c) * K;
-        v.x = Mn[rfc(n, m)] * (m == 0 ? 0.70710678118654752 : 1.0);
-        if (m > 0) v.y = Mn[rfs(n, m)];
+    const int64_t total = (count + 1) * per, step = static_cast<int64_t>(gridDim.x) * 256;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += step) {
+        const int64_t node = i / per;
+        const int k = static_cast<int>(i - node * per);
+        const int pr = k / nc, c = k - pr * nc;
+        int n = static_cast<int>((sqrtf(8.0f * pr + 1.0f) - 1.0f) * 0.5f);
+        while ((n + 1) * (n + 2) / 2 <= pr) ++n;
+        while (n * (n + 1) / 2 > pr) --n;
+        const int m = pr - n * (n + 1) / 2;
+        double2 v{0.0, 0.0};
+        if (node < count) {
+            const double* Mn = M + (node * nc + c) * K;
+            v.x = Mn[rfc(n, m)] * (m == 0 ? 0.70710678118654752 : 1.0);
+            if (m > 0) v.y = Mn[rfs(n, m)];
+        }
+        Mx[i] = v;
     }
-    Mx[i] = v;
 }
 
 // ------------------------------------------------------------------ L2P
@@ -1009,7 +1010,9 @@ void launch_pair_copy(const double* M, int64_t count, int nc, int p, double* Mx,
 {
     const int np = (p + 1) * (p + 2) / 2;
     const int64_t total = (count + 1) * np * nc;
-    hipLaunchKernelGGL(pair_copy_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s, M, count, nc,
+    // a launch takes fewer than 2^32 threads, which p = 12 would pass at 11.8M nodes
+    const int64_t blocks = std::min<int64_t>((total + 255) / 256, int64_t(1) << 23);
+    hipLaunchKernelGGL(pair_copy_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, M, count, nc,
                        np, (p + 1) * (p + 1), reinterpret_cast<double2*>(Mx), stamp);
 }
 
