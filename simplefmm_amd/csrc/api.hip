@@ -1502,31 +1502,29 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
     // (One limit of 2^18 pairs for every tree left a few wavefronts working
     // alone: 200k Plummer, 1 component, 1.70 -> 0.37 ms; 5k uniform, curl, 172 ->
     // 24 us; 20k Plummer mixed 460 -> 105 us; 16M Plummer 14.5 -> 13.9 ms.)
+    std::vector<int64_t> l_total(nleaf), l_per(nleaf), l_nitem(nleaf), l_item0(nleaf + 1, 0), l_row0(nleaf + 1, 0),
+        l_split0(nleaf + 1, 0);
     std::atomic<int64_t> all_pairs{0};
     parallel_ranges(nleaf, nthreads, [&](int64_t g0, int64_t g1, int) {
         int64_t sum = 0;
-        for (int64_t g = g0; g < g1; ++g) {
-            int64_t total = 0;
-            for (int64_t r = t.near_row[g]; r < t.near_row[g + 1]; ++r) total += t.near_end[r] - t.near_begin[r];
-            sum += total * std::max<int64_t>(lf_end[g] - lf_begin[g], 16);
-        }
-        all_pairs += sum;
-    });
-    const int64_t most = std::min<int64_t>(int64_t(1) << 18, std::max<int64_t>(nleaf >= 4096 ? 1 << 14 : 1 << 12, all_pairs / (1024 * 16)));
-    std::vector<int64_t> l_total(nleaf), l_per(nleaf), l_nitem(nleaf), l_item0(nleaf + 1, 0), l_row0(nleaf + 1, 0),
-        l_split0(nleaf + 1, 0);
-    parallel_ranges(nleaf, nthreads, [&](int64_t g0, int64_t g1, int) {
         for (int64_t g = g0; g < g1; ++g) {
             int64_t total = 0;
             for (int64_t r = t.near_row[g]; r < t.near_row[g + 1]; ++r) {
                 near_pref[r] = total;
                 total += t.near_end[r] - t.near_begin[r];
             }
-            const int64_t nt = lf_end[g] - lf_begin[g];
+            l_total[g] = total;
+            sum += total * std::max<int64_t>(lf_end[g] - lf_begin[g], 16);
+        }
+        all_pairs += sum;
+    });
+    const int64_t most = std::min<int64_t>(int64_t(1) << 18, std::max<int64_t>(nleaf >= 4096 ? 1 << 14 : 1 << 12, all_pairs / (1024 * 16)));
+    parallel_ranges(nleaf, nthreads, [&](int64_t g0, int64_t g1, int) {
+        for (int64_t g = g0; g < g1; ++g) {
+            const int64_t total = l_total[g], nt = lf_end[g] - lf_begin[g];
             const int64_t per = std::max<int64_t>(64, most / std::max<int64_t>(nt, 16) / 64 * 64);
             l_per[g] = total * std::max<int64_t>(nt, 16) * 2 <= 3 * most ? total : per;
             l_nitem[g] = l_per[g] > 0 ? (total + l_per[g] - 1) / l_per[g] : 1;
-            l_total[g] = total;
         }
     });
     for (int64_t g = 0; g < nleaf; ++g) {
@@ -1641,7 +1639,7 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
         // first (20k Plummer p = 12, ~200 blocks: 0.49 ms against 0.67 with 8); beyond, 8
         // share each operator among twice the columns (4M uniform p = 10: 25.6 against 33.8).
         int64_t blocks16 = 0;
-        for (int l = 2; l <= D; ++l) {
+        for (int l = 2; l <= D && blocks16 <= 256; ++l) {
             int64_t nodes[8] = {};
             for (int32_t a = 0; a < t.lv[l].n_node(); ++a) ++nodes[t.lv[l].code[a] & 7];
             for (int64_t c : nodes) blocks16 += (c + 15) / 16;
