@@ -17,7 +17,7 @@
 //     the 16 columns of 16x16x32 f16 MFMA tiles;
 //   * the offsets present in the block are walked grouped by azimuth: the
 //     sources' columns are rotated by e^{i m phi} in FP32 registers and scaled
-//     (the largest value over the wavefront's sources to below 2^15), split as
+//     (the largest value of a column's sources to below 2^15), split as
 //     x = H + L with H = f16(x), L = f16(x - H), and C += A_hi H + A_lo H +
 //     A_hi L runs on the f16 matrix cores with FP32 accumulation; D_c, scaled
 //     to the f16 range and split the same way, is copied into LDS by the LDS
@@ -365,10 +365,12 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
     const int64_t e0 = a.blk_row[blk];
     const int ne = static_cast<int>(a.blk_row[blk + 1] - e0);
 
-    // scale of this wavefront's columns (the components of neighbouring
-    // targets): the largest |value| over their sources maps below 2^15, so
-    // rotated values stay below 2^15.5 < 65504 and keep 22 bits down to 2^-18
-    // of the largest; one value per wavefront keeps the azimuth factors scalar
+    // scale of this lane's column (one component of one target): the largest
+    // |value| over its sources maps below 2^15, so rotated values stay below
+    // 2^15.5 < 65504 and keep 22 bits down to 2^-18 of the largest.  A scale shared
+    // by several components would take those bits from the smaller ones, which
+    // differ by any factor (the caller's charges; potential and gradient by the
+    // length unit).  The four lanes of a column take the same
     float mx = 0.0f;
     if (tg >= 0 && q == 0) {
         for (int i0 = 0; i0 < ne; i0 += 8) {
@@ -380,14 +382,13 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
                 if (sn[u] >= 0) mx = fmaxf(mx, a.nodemax[static_cast<int64_t>(sn[u]) * NC + comp]);
         }
     }
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    for (int o = 32; o > 8; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
     int sexp = 0;
     if (mx > 0.0f) {
         int ex;
         (void)frexpf(mx, &ex);  // mx < 2^ex
-        sexp = 15 - ex;
+        sexp = min(15 - ex, 127);  // a finite scale also for the smallest FP32 values
     }
-    sexp = __builtin_amdgcn_readfirstlane(sexp);
     const float sc = ldexpf(1.0f, sexp);
     const float neg1 = dense_neg1();
     // a wave-uniform float held in a scalar register
@@ -443,11 +444,11 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
         });
     }
     __syncthreads();  // saz, smeta, srow_*
-    float csx[P + 1], csy[P + 1];  // cos, sin of m phi of the current azimuth group, times sc
+    float csx[P + 1], csy[P + 1];  // cos, sin of m phi of the current azimuth group
     auto factors = [&](int g) {
         for (int m = 0; m <= P; ++m) {
-            csx[m] = uniform(saz[(g * (P + 1) + m) * 2] * sc);
-            csy[m] = uniform(saz[(g * (P + 1) + m) * 2 + 1] * sc);
+            csx[m] = uniform(saz[(g * (P + 1) + m) * 2]);
+            csy[m] = uniform(saz[(g * (P + 1) + m) * 2 + 1]);
         }
     };
     int i = 0, g = -1;
@@ -514,10 +515,14 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
                 float cm = csx[m], sm = csy[m];
                 if constexpr (z != 0 && m != 0) {  // lane groups whose element is of order 0
                     const bool zq = (z >> qv) & 1;
-                    cm = zq ? sc : cm;
+                    cm = zq ? 1.0f : cm;
                     sm = zq ? 0.0f : sm;
                 }
-                const float xrj = xr[ks][j], xij = xi[ks][j];
+                // the scale, a power of two: exact.  (On the columns, 16 multiplies per
+                // K-step and 1% of the evaluation: 4M uniform p = 10 30.7 -> 31.1 ms, 16M
+                // Plummer p = 12 126.0 -> 127.6.  One scale per wavefront would go into
+                // the azimuth factors.)
+                const float xrj = xr[ks][j] * sc, xij = xi[ks][j] * sc;
                 _Float16 hh, ll;
                 dense_split(__builtin_fmaf(xrj, cm, -(xij * sm)), hh, ll, neg1);
                 bch[B][j] = hh;
