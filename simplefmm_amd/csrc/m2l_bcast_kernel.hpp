@@ -41,8 +41,8 @@ __host__ __device__ constexpr int row_of(int mode, int n, int m, int part)
 
 // c += op[lane LN of this lane's 16-lane row] * x.  The compiler does not form
 // this instruction from v_mov_b64_dpp and v_fma_f64, hence the asm.  A DPP read
-// needs two wait states after a vector write of op: op comes from memory, and
-// settle() separates it from any register copy.
+// needs two wait states after a vector write of op: op comes from memory, and an
+// s_nop at the start of a step separates it from any register copy before.
 template <int LN>
 __device__ __forceinline__ void fmac_row(double& c, double op, double x)
 {
@@ -352,8 +352,8 @@ __device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t g, int64_
                 for (int k = 0; k < WV::NR; ++k)
                     if (st > 0) wv.rot.v[k] = wv.bank.v[k];
                 load_ops<WV::NT>(wv.bank.v, cox_ops(w), lane);
-                asm volatile("s_nop 1");
             }
+            asm volatile("s_nop 1");  // in every step: a copy may end the step before, too
             __builtin_amdgcn_sched_barrier(0);
             change = cls_of(wn) != cls_of(w);
             wv.stage1(X, lane, f.x, f.y);
