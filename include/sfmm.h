@@ -198,7 +198,8 @@ typedef struct {
  * (largest first) and captures the launch sequence into a HIP graph that every
  * launch replays.  streams: 1..8, or 0 to tune first (into scratch outputs): the
  * tile shapes of each expansion order on its largest problem (as
- * sfmm_plan_tune; set on every plan of that order), then 1, 2, 4, 8 streams and
+ * sfmm_plan_tune; set on every plan of that order, the M2L's apart for the plans
+ * whose shape before any tuning is 4 and 8), then 1, 2, 4, 8 streams and
  * every item on its plan's own stream, each timed as graph replays, keeping the
  * fastest.  The items' arrays must stay valid while the batch is used; a batch
  * keeps the tile shapes its plans had when it was created. */

@@ -252,6 +252,7 @@ struct sfmm_plan_s {
     int dense_op_exp = 0;
     int dense_kd = 0;                   // floats per (node, component) of the FP32 copy
     int dense_waves = 8;                // the dense M2L's tile shape: wavefronts per workgroup (4, 8)
+    int dense_default = 8;              // the shape that the tree's size gives
     std::vector<int32_t> dense_grp;     // azimuth group per offset id
     sfmm::SelfCorr self;                // self-list corrections (empty without a self generator)
     std::vector<int64_t> slist_row, slist_val;  // far self pairs per particle, original order (_slist)
@@ -1071,8 +1072,9 @@ int batch_capture(sfmm_batch_s* B, const std::vector<sfmm_batch_item>& items, co
 // stream s and keeps the fastest: the near field's targets per lane (1, 2, 4;
 // near field alone) when `near`, the dense M2L's wavefronts per workgroup (8, 4;
 // far field alone) when `far` and the plan uses it.  Each shape is timed as the
-// best of three runs after a warm-up; a shape other than the default (2 and 8)
-// is kept only when at least 2% faster.  The plan must be prepared for `it`.
+// best of three runs after a warm-up; a shape other than the default (2, and the
+// plan's dense_default) is kept only when at least 2% faster.  The plan must be
+// prepared for `it`.
 int tune_tiles(sfmm_plan_s* P, const sfmm_batch_item& it, hipStream_t s, bool near, bool far, int* tpl_out,
                int* waves_out)
 {
@@ -1117,9 +1119,9 @@ int tune_tiles(sfmm_plan_s* P, const sfmm_batch_item& it, hipStream_t s, bool ne
         if (tpl_out) *tpl_out = best_tpl;
     }
     if (far && P->dense && rc == SFMM_OK) {
-        int best_w = 8;
+        int best_w = P->dense_default;
         float best_ms = -1.0f;
-        for (int w : {8, 4}) {
+        for (int w : {P->dense_default, 12 - P->dense_default}) {
             set_dense_waves(P, w);
             if ((rc = prepare(P, it.kind, it.ncharge, it.which, mode, qdim, nc)) != SFMM_OK) break;
             float ms = 0.0f;
@@ -1644,7 +1646,7 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
             for (int32_t a = 0; a < t.lv[l].n_node(); ++a) ++nodes[t.lv[l].code[a] & 7];
             for (int64_t c : nodes) blocks16 += (c + 15) / 16;
         }
-        P->dense_waves = blocks16 <= 256 ? 4 : 8;
+        P->dense_waves = P->dense_default = blocks16 <= 256 ? 4 : 8;
         const uint16_t* dops = nullptr;
         const float* dmax = nullptr;
         if ((rc = P->upload(ops, &dops)) || (rc = P->upload(az, &P->dense_az)) ||
@@ -2034,30 +2036,32 @@ int sfmm_batch_create(const sfmm_batch_item* items, int count, int streams, sfmm
             }
             return SFMM_OK;
         };
-        // tile shapes (near field, dense M2L) of each expansion order, timed on its
-        // largest problem and set on every plan of that order
+        // tile shapes of each expansion order, timed on its largest problem and set on
+        // every plan of that order; the dense M2L's apart for the plans of either
+        // default, which small and large trees differ in
         std::vector<int> orders;
         for (const auto& it : B->items)
             if (std::find(orders.begin(), orders.end(), it.plan->p) == orders.end()) orders.push_back(it.plan->p);
         for (int p : orders) {
-            int big = -1, big_dense = -1;
+            int big = -1, big_dense[2] = {-1, -1};  // by default shape: 8, 4 wavefronts
             for (int i = 0; i < count; ++i) {
                 const sfmm_plan_s* Q = B->items[i].plan;
                 if (Q->p != p) continue;
                 if (big < 0 || Q->tree->t.n > B->items[big].plan->tree->t.n) big = i;
-                if (Q->dense && (big_dense < 0 || Q->tree->t.n > B->items[big_dense].plan->tree->t.n)) big_dense = i;
+                int& bd = big_dense[Q->dense_default == 4];
+                if (Q->dense && (bd < 0 || Q->tree->t.n > B->items[bd].plan->tree->t.n)) bd = i;
             }
-            int tpl = 2, waves = 8;
+            int tpl = 2, waves[2] = {8, 4};
             if ((rc = tune_tiles(B->items[big].plan, trial[big], s0, true, false, &tpl, nullptr)) != SFMM_OK) break;
-            if (big_dense >= 0 &&
-                (rc = tune_tiles(B->items[big_dense].plan, trial[big_dense], s0, false, true, nullptr, &waves)) != SFMM_OK)
-                break;
+            for (int k = 0; k < 2 && rc == SFMM_OK; ++k)
+                if (const int i = big_dense[k]; i >= 0)
+                    rc = tune_tiles(B->items[i].plan, trial[i], s0, false, true, nullptr, &waves[k]);
             for (int i = 0; i < count && rc == SFMM_OK; ++i) {
                 sfmm_plan_s* Q = B->items[i].plan;
                 if (Q->p != p) continue;
                 Q->p2p_tpl = tpl;
                 if (!Q->dense) continue;
-                set_dense_waves(Q, waves);
+                set_dense_waves(Q, waves[Q->dense_default == 4]);
                 sfmm::Mode mode;
                 int qdim, nc;
                 rc = prepare(Q, B->items[i].kind, B->items[i].ncharge, B->items[i].which, mode, qdim, nc);
