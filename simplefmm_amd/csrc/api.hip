@@ -68,7 +68,8 @@ int fail(int code, const std::string& msg)
 // Every device allocation of the library goes through here.  Fault injection
 // for tests: while the environment variable SFMM_FAULT_ALLOC holds a count k,
 // the first k allocations after it was set (or changed) succeed and every
-// later one fails as if the device were out of memory.
+// later one fails as if the device were out of memory; while SFMM_FAULT_ALLOC_BYTES
+// is set, every allocation of more bytes does.
 hipError_t dev_malloc(void** p, size_t bytes)
 {
     static std::mutex mu;
@@ -88,7 +89,13 @@ hipError_t dev_malloc(void** p, size_t bytes)
         std::lock_guard<std::mutex> lock(mu);
         armed.clear();
     }
-    return hipMalloc(p, bytes);
+    const char* limit = std::getenv("SFMM_FAULT_ALLOC_BYTES");
+    const hipError_t e = limit && bytes > std::strtoull(limit, nullptr, 10) ? hipErrorOutOfMemory : hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();  // the caller handles it; a launch's check must not find it
+    }
+    return e;
 }
 template <class T>
 hipError_t dev_malloc(T** p, size_t bytes)
@@ -208,7 +215,7 @@ struct sfmm_plan_s {
     std::vector<void*> owned;
     std::vector<int64_t> level_first;  // gnode of the first node of each level (size depth+2)
     double* M = nullptr;
-    double* L = nullptr;
+    double* L = nullptr;   // M itself where the M2L reads a copy of the multipoles only (bcast)
     float* M32 = nullptr;  // FP32 copy of M for the mixed-precision M2L
     int nc_alloc = 0;
     double* qbuf = nullptr;
@@ -236,8 +243,17 @@ struct sfmm_plan_s {
     // FP64: M2L with broadcast operators (m2l_bcast.hpp)
     bool bcast = false;
     sfmm::BcastArgs bc;                 // operators and azimuths
-    sfmm::BcastArgs bcg[5];             // with the work lists, per component count (built on first use)
+    struct BcastWork {
+        sfmm::BcastArgs args;           // all spans' workgroups
+        struct Span {
+            int64_t node0, nodes;       // whose multipoles are copied before
+            int64_t item0, items;       // and the workgroups then launched
+        };
+        std::vector<Span> span;         // all levels, or (by_level) one per level
+        bool by_level = false;
+    } bcg[5];                           // work lists per component count (built on first use)
     double* Mx = nullptr;               // its copy of the multipoles
+    bool mx_by_level = false;           // holds one level's at a time
     const double* zero_cols = nullptr;  // 4 (p+1)^2 zeros: M2L columns of absent sources
     const double* m2m_frag = nullptr;   // matrix-core M2M / L2L operators [8][nfrag][64]
     const double* l2l_frag = nullptr;
@@ -266,8 +282,8 @@ struct sfmm_plan_s {
     ~sfmm_plan_s()
     {
         for (void* p : owned) (void)hipFree(p);
+        if (L != M) (void)hipFree(L);
         (void)hipFree(M);
-        (void)hipFree(L);
         (void)hipFree(M32);
         (void)hipFree(Mx);
         (void)hipFree(qbuf);
@@ -361,13 +377,24 @@ int mode_of(int kind, int ncharge, sfmm::Mode& mode, int& qdim, int& nc)
     }
 }
 
+// Nodes of the copy of the multipoles that the broadcast M2L reads: all from level 2
+// on, or (by_level) the fullest level's, and one of zeros.
+int64_t bcast_copy_nodes(const sfmm_plan_s* P, bool by_level)
+{
+    const int D = P->tree->t.depth;
+    if (D < 2) return 1;
+    int64_t most = 0;
+    for (int l = 2; l <= D; ++l) most = std::max(most, P->level_first[l + 1] - P->level_first[l]);
+    return (by_level ? most : P->level_first[D + 1] - P->level_first[2]) + 1;
+}
+
 int ensure_buffers(sfmm_plan_s* P, int nc, int qdim)
 {
     const int64_t nnode = P->level_first.back();
     const int64_t n = P->tree->t.n;
     if (nc > P->nc_alloc) {
+        if (P->L != P->M) (void)hipFree(P->L);
         (void)hipFree(P->M);
-        (void)hipFree(P->L);
         (void)hipFree(P->M32);
         (void)hipFree(P->Mx);
         P->M = P->L = nullptr;
@@ -375,8 +402,14 @@ int ensure_buffers(sfmm_plan_s* P, int nc, int qdim)
         P->Mx = nullptr;
         P->nc_alloc = 0;
         const size_t bytes = sizeof(double) * static_cast<size_t>(nnode) * nc * P->K;
-        if (dev_malloc(&P->M, bytes) != hipSuccess || dev_malloc(&P->L, bytes) != hipSuccess)
+        if (dev_malloc(&P->M, bytes) != hipSuccess) return fail(SFMM_ERR_ALLOC, "hipMalloc failed (expansions)");
+        if (P->bcast) {
+            // the M2L's kernels read the copy, so that the local expansions can take the
+            // multipoles' place: every evaluation writes all of M, then all of L
+            P->L = P->M;
+        } else if (dev_malloc(&P->L, bytes) != hipSuccess) {
             return fail(SFMM_ERR_ALLOC, "hipMalloc failed (expansions)");
+        }
         if (P->precision == SFMM_MIXED && P->m2l_kernel == 0) {
             // the dense layout pads each (node, component) to dense_kd floats
             // (the FP32 copy kernel writes the padding as zeros)
@@ -386,8 +419,15 @@ int ensure_buffers(sfmm_plan_s* P, int nc, int qdim)
             HIP_TRY(hipMemset(P->M32, 0, b32));
         }
         if (P->bcast) {
-            const size_t bx = sizeof(double) * static_cast<size_t>(nnode + 1) * nc * 2 * sfmm::bcast_pairs(P->p);
-            if (dev_malloc(&P->Mx, bx) != hipSuccess) return fail(SFMM_ERR_ALLOC, "hipMalloc failed (multipole copy)");
+            // the copy of all levels, or, where memory is short, of one at a time
+            const size_t per = sizeof(double) * static_cast<size_t>(nc) * 2 * sfmm::bcast_pairs(P->p);
+            P->mx_by_level = dev_malloc(&P->Mx, per * bcast_copy_nodes(P, false)) != hipSuccess;
+            if (P->mx_by_level) {
+                if (dev_malloc(&P->Mx, per * bcast_copy_nodes(P, true)) != hipSuccess)
+                    return fail(SFMM_ERR_ALLOC, "hipMalloc failed (multipole copy)");
+                for (auto& w : P->bcg)  // lists for the copy of all levels (a batch may still hold them)
+                    if (!w.by_level) w = {};
+            }
         }
         P->nc_alloc = nc;
     }
@@ -596,15 +636,16 @@ int build_m2l_blocks(sfmm_plan_s* P, int nc)
 // octants of each z half form a group of four rows.  A group's steps go class
 // by class; within a class, step k holds each row's k-th present offset, so a
 // class takes as many steps as its fullest row (full rows of one z half have
-// equal counts: x and y reflections keep the polar class).
-int build_bcast_groups(sfmm_plan_s* P, int nc)
+// equal counts: x and y reflections keep the polar class).  by_level: the levels run
+// one after another, each behind the copy of its multipoles, and no group is cut.
+int build_bcast_groups(sfmm_plan_s* P, int nc, bool by_level)
 {
-    if (P->bcg[nc].grp_tgt || P->tree->t.depth < 2) return SFMM_OK;
     const sfmm::Tree& t = P->tree->t;
     const int TB = 16 / nc;
     const auto& cls = P->tables.off_class;
     const auto& d2 = P->tables.off_d2;
-    const int32_t zero_node = static_cast<int32_t>(P->level_first.back());
+    // the node of zeros follows the copied ones
+    auto zero_node = [&](int l) { return static_cast<int32_t>(by_level ? P->level_first[l + 1] : P->level_first.back()); };
     std::vector<std::vector<int>> class_off(70);
     for (int off = 0; off < 343; ++off)
         if (cls[off] >= 0) class_off[cls[off]].push_back(off);
@@ -672,7 +713,7 @@ int build_bcast_groups(sfmm_plan_s* P, int nc)
             std::fill(used.begin(), used.end(), 0);
             visit(G, [&](int off, int r, int tt, int32_t s) {
                 int32_t* c = cols.data() + (static_cast<size_t>(off) * 4 + r) * TB;
-                if (!(used[off] >> r & 1)) std::fill(c, c + TB, zero_node);
+                if (!(used[off] >> r & 1)) std::fill(c, c + TB, zero_node(G.level));
                 used[off] |= 1 << r;
                 c[tt] = static_cast<int32_t>(first + s);
             });
@@ -695,7 +736,7 @@ int build_bcast_groups(sfmm_plan_s* P, int nc)
                     for (int off : offs) k += used[off] >> r & 1;
                     for (; k < steps; ++k) {  // this row has no offset left in the class
                         meta[(st + k) * 4 + r] = offs[0] | cls[offs[0]] << 9 | d2[offs[0]] << 16;
-                        std::fill_n(src.data.get() + ((st + k) * 4 + r) * TB, TB, zero_node);
+                        std::fill_n(src.data.get() + ((st + k) * 4 + r) * TB, TB, zero_node(G.level));
                     }
                 }
                 st += steps;
@@ -706,36 +747,48 @@ int build_bcast_groups(sfmm_plan_s* P, int nc)
     // groups are dealt to the XCDs in contiguous shares of equal steps, so that
     // neighbours share an L2, and cut into runs towards the end of a share
     std::vector<int64_t> item, split;
-    std::vector<std::array<int64_t, 4>> share[8];
     int64_t rows = 0;
-    const int64_t total = grp_row[ng];
-    for (int x = 0; x < 8; ++x) {
+    sfmm_plan_s::BcastWork W;
+    W.by_level = by_level;
+    int64_t ga = 0, gb = 0;
+    for (int l = 2; l <= t.depth; ++l) {
+        while (gb < ng && groups[gb].level == l) ++gb;
+        if (!by_level && l < t.depth) continue;
+        const int64_t first = by_level ? P->level_first[l] : P->level_first[2];
+        W.span.push_back({first, P->level_first[l + 1] - first, static_cast<int64_t>(item.size()) / 4, 0});
+        // groups [ga, gb)
+        const int64_t base = grp_row[ga], total = grp_row[gb] - base;
         auto first_at = [&](int64_t step) {  // first group at or after a step
-            return std::lower_bound(grp_row.begin(), grp_row.begin() + ng, step) - grp_row.begin();
+            return std::lower_bound(grp_row.begin() + ga, grp_row.begin() + gb, base + step) - grp_row.begin();
         };
-        const int64_t g0 = x == 0 ? 0 : first_at(total * x / 8), g1 = x == 7 ? ng : first_at(total * (x + 1) / 8);
-        for (int64_t g = g0; g < g1; ++g) {
-            const int64_t r0 = grp_row[g], n = grp_row[g + 1] - r0;
-            const int64_t most = sfmm::bcast_run_steps(P->p, grp_row[g1] - r0, total);
-            const int64_t runs = 2 * n > 3 * most ? (n + most - 1) / most : 1;
-            for (int64_t k = 0; k < runs; ++k)
-                share[x].push_back({g, r0 + n * k / runs, r0 + n * (k + 1) / runs, runs > 1 ? rows + k : -1});
-            if (runs > 1) {
-                split.insert(split.end(), {g, rows, runs});
-                rows += runs;
+        std::vector<std::array<int64_t, 4>> share[8];
+        for (int x = 0; x < 8; ++x) {
+            const int64_t g0 = x == 0 ? ga : first_at(total * x / 8), g1 = x == 7 ? gb : first_at(total * (x + 1) / 8);
+            for (int64_t g = g0; g < g1; ++g) {
+                const int64_t r0 = grp_row[g], n = grp_row[g + 1] - r0;
+                const int64_t most = sfmm::bcast_run_steps(P->p, grp_row[g1] - r0, total);
+                const int64_t runs = !by_level && 2 * n > 3 * most ? (n + most - 1) / most : 1;
+                for (int64_t k = 0; k < runs; ++k)
+                    share[x].push_back({g, r0 + n * k / runs, r0 + n * (k + 1) / runs, runs > 1 ? rows + k : -1});
+                if (runs > 1) {
+                    split.insert(split.end(), {g, rows, runs});
+                    rows += runs;
+                }
             }
         }
+        size_t longest = 0;
+        for (const auto& sh : share) longest = std::max(longest, sh.size());
+        for (size_t k = 0; k < longest; ++k)
+            for (const auto& sh : share) {
+                const std::array<int64_t, 4> none{-1, 0, 0, -1};
+                const auto& it = k < sh.size() ? sh[k] : none;
+                item.insert(item.end(), it.begin(), it.end());
+            }
+        W.span.back().items = static_cast<int64_t>(item.size()) / 4 - W.span.back().item0;
+        ga = gb;
     }
-    size_t longest = 0;
-    for (const auto& sh : share) longest = std::max(longest, sh.size());
-    for (size_t k = 0; k < longest; ++k)
-        for (const auto& sh : share) {
-            const std::array<int64_t, 4> none{-1, 0, 0, -1};
-            const auto& it = k < sh.size() ? sh[k] : none;
-            item.insert(item.end(), it.begin(), it.end());
-        }
-    sfmm::BcastArgs A = P->bc;
-    A.n_item = static_cast<int64_t>(item.size()) / 4;
+    sfmm::BcastArgs& A = W.args;
+    A = P->bc;
     A.n_split = static_cast<int64_t>(split.size()) / 3;
     int rc;
     if ((rc = P->upload(tgt, &A.grp_tgt)) || (rc = P->upload(item, &A.item)) || (rc = P->upload(split, &A.split)) ||
@@ -750,8 +803,21 @@ int build_bcast_groups(sfmm_plan_s* P, int nc)
         A.partial = static_cast<double*>(part);
         A.n_partial = rows;
     }
-    P->bcg[nc] = A;
+    P->bcg[nc] = std::move(W);
     return SFMM_OK;
+}
+
+// The broadcast M2L's work lists; by level, without partial sums, where memory is short.
+int ensure_bcast_groups(sfmm_plan_s* P, int nc)
+{
+    if (P->bcg[nc].args.grp_tgt || P->tree->t.depth < 2) return SFMM_OK;
+    const size_t owned = P->owned.size();
+    int rc = build_bcast_groups(P, nc, P->mx_by_level);
+    if (rc == SFMM_ERR_ALLOC && !P->mx_by_level) {
+        for (; P->owned.size() > owned; P->owned.pop_back()) (void)hipFree(P->owned.back());
+        rc = build_bcast_groups(P, nc, true);
+    }
+    return rc;
 }
 
 // M2M and L2L work lists of every level: blocks of 16/nc parents, each with one
@@ -817,10 +883,12 @@ int build_translate_blocks(sfmm_plan_s* P, int nc)
     }
     if (most > 0) {
         void* part = nullptr;
-        if (dev_malloc(&part, sizeof(double) * static_cast<size_t>(most) * 8 * P->K * 16) != hipSuccess)
-            return fail(SFMM_ERR_ALLOC, "hipMalloc failed (M2M partial sums)");
+        // where memory is short, of fewer blocks at a time
+        while (dev_malloc(&part, sizeof(double) * static_cast<size_t>(most) * 8 * P->K * 16) != hipSuccess)
+            if ((most /= 2) == 0) return fail(SFMM_ERR_ALLOC, "hipMalloc failed (M2M partial sums)");
         P->owned.push_back(part);
         A.part = static_cast<double*>(part);
+        A.part_blocks = most;
     }
     sfmm::TransArgs B = A;  // published together once every upload succeeded
     A.frag = P->m2m_frag;
@@ -848,7 +916,7 @@ int prepare(sfmm_plan_s* P, int kind, int ncharge, int which, sfmm::Mode& mode, 
     if (int rc = ensure_buffers(P, nc, qdim)) return rc;
     if (P->m2l_kernel == 0) {
         if (int rc = P->dense   ? build_dense_blocks(P, nc)
-                     : P->bcast ? build_bcast_groups(P, nc)
+                     : P->bcast ? ensure_bcast_groups(P, nc)
                                 : build_m2l_blocks(P, nc))
             return rc;
         if (int rc = build_translate_blocks(P, nc)) return rc;
@@ -907,12 +975,17 @@ int run_on(sfmm_plan_s* P, sfmm::Mode mode, int nc, int qdim, const double* dQ, 
                                    P->dense ? P->dense_nodemax + f2 * nc : nullptr, stamp(3), s);
         }
         if (P->bcast) {
-            const int64_t f2 = P->level_first[2], pr = 2 * sfmm::bcast_pairs(P->p);
-            sfmm::launch_pair_copy(P->M + f2 * nc * P->K, P->level_first.back() - f2, nc, P->p, P->Mx + f2 * nc * pr, stamp(3),
-                                   s);
-            sfmm::BcastArgs A = P->bcg[nc];
-            A.Mx = P->Mx;
-            sfmm::launch_m2l_bcast(A, P->p, nc, P->L, s);
+            const sfmm_plan_s::BcastWork& W = P->bcg[nc];
+            for (const auto& sp : W.span) {
+                sfmm::launch_pair_copy(P->M + sp.node0 * nc * P->K, sp.nodes, nc, P->p, P->Mx,
+                                       &sp == W.span.data() ? stamp(3) : nullptr, s);
+                sfmm::BcastArgs A = W.args;
+                A.Mx = P->Mx;
+                A.node0 = sp.node0;
+                A.item += 4 * sp.item0;
+                A.n_item = sp.items;
+                sfmm::launch_m2l_bcast(A, P->p, nc, P->L, s);
+            }
         } else if (P->dense) {
             sfmm::launch_m2l_dense(P->dns[nc], P->p, nc, M32, P->L, s);
         } else if (P->m2l_kernel == 0) {

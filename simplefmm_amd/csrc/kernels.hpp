@@ -113,7 +113,9 @@ struct BcastArgs {
     const double* coax = nullptr;        // [28][registers][16] coaxial elements
     const double* az_fwd = nullptr;      // [343][16] (cos m phi - 1, sin m phi), m = 1..16
     const double* az_back = nullptr;     // [343][16] (cos m phi, sin m phi)
-    const double* Mx = nullptr;          // multipoles, [gnode][pair (n, m)][nc][Re, Im] (order 0 / sqrt 2) + one zero node
+    // multipoles, [gnode - node0][pair (n, m)][nc][Re, Im] (order 0 / sqrt 2) + one zero node; L may be what they were copied from
+    const double* Mx = nullptr;
+    int64_t node0 = 0;
     const double *rot_sin = nullptr, *coax_sin = nullptr;  // p > 13: rot and coax hold the cos blocks, these the sin
     int64_t n_partial = 0;
     double* partial = nullptr;           // [n_partial, p > 13: cos then sin][(p+1)^2][64]
@@ -161,8 +163,9 @@ struct TransArgs {
     const int32_t* ent_oct = nullptr;   // child octant per entry
     const int32_t* ent_node = nullptr;  // [entries][16/nc] child gnodes, -1 = none
     const double* frag = nullptr;      // [8][nfrag][64]
-    // M2M partial sums of a split level, [block < kTrSplitChunk][8][(p+1)^2][16]
+    // M2M partial sums of a split level, part_blocks (<= kTrSplitChunk) at a time: [block][8][(p+1)^2][16]
     double* part = nullptr;
+    int64_t part_blocks = 0;
 };
 // Levels of at most this many blocks run one workgroup per entry instead of one
 // per block.  M2M: below it the blocks leave compute units idle, above it the

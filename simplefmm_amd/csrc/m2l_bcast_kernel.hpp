@@ -320,7 +320,7 @@ __device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t g, int64_
 #pragma unroll
     for (int k = 0; k < (WV::NCOL > 0 ? WV::NCOL : 1); ++k) wv.are[k] = wv.aim[k] = 0.0;
 
-    const D2* Mx = reinterpret_cast<const D2*>(a.Mx) + comp;
+    const D2* Mx = reinterpret_cast<const D2*>(a.Mx) + comp - a.node0 * (NP * NC);
     // steps are counted from s0 in 32 bits
     const int ns = static_cast<int>(s1 - s0);
     const int32_t* srcs = a.step_src + s0 * (4 * TB) + row * TB + t;

@@ -326,7 +326,7 @@ void translate_nc(const TransArgs& a, LevelSpan b, int nc, double* io, hipStream
 {
     constexpr int64_t most = tr_split_most(P, UPPER);
     if (b.count <= most) {
-        const int64_t chunk = UPPER ? b.count : kTrSplitChunk;
+        const int64_t chunk = UPPER ? b.count : a.part_blocks;
         for (int64_t at = 0; at < b.count; at += chunk) {
             const int64_t first = b.first + at, count = b.count - at < chunk ? b.count - at : chunk;
             hipLaunchKernelGGL((translate_split_kernel<P, UPPER>), dim3(static_cast<unsigned>(count), 8),
