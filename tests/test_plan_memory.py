@@ -97,3 +97,32 @@ def test_component_counts_before_and_after_memory_got_short(monkeypatch):
         monkeypatch.delenv("SFMM_FAULT_ALLOC_BYTES", raising=False)
         print(f"n={n} p={p} ncharge={nq}: {rel_l2(u, ref[k]):.1e}", flush=True)
         assert rel_l2(u, ref[k]) < TOLERANCE
+
+
+def test_near_field_of_fat_leaves_takes_no_more_partial_sums():
+    # 1562 targets to a leaf: runs of 128 sources (2^18 pairs) and 191 runs to a leaf
+    # on average, 32 bytes per target and run: 0.61 GB
+    import torch
+    n = 100_000
+    rng = np.random.default_rng(7)
+    pos, Q = rng.uniform(size=(n, 3)), rng.uniform(-1, 1, (n, 1))
+    part = api.OctreePartitioner(pos, api.Box(corner=[0.0, 0.0, 0.0], width=1.0)).refine(20, 2000)
+    fmm = api.FMM3D(part, 2, ncharge=1)
+    dq = torch.from_numpy(Q).cuda()
+    du = torch.zeros((n, 4), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    fmm.evaluate_device(api.POTGRAD, 1, dq.data_ptr(), du.data_ptr(), api.NEAR)
+    fmm.synchronize()
+    used = before - torch.cuda.mem_get_info()[0]
+    print(f"n={n}: {used / 1e9:.2f} GB", flush=True)
+    assert used < 0.7e9
+    tg = np.arange(0, n, 997)
+    got = du.cpu().numpy()
+    for i in tg[:20]:
+        src = part.near_sources(i)
+        src = src[src != i]
+        d = pos[i] - pos[src]
+        r = np.sqrt((d * d).sum(1))
+        scale = (np.abs(Q[src, 0]) / r).sum()
+        assert abs(got[i, 0] - (Q[src, 0] / r).sum()) <= 1e-12 * scale
