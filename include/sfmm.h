@@ -150,7 +150,10 @@ int sfmm_plan_set_tiles(sfmm_plan plan, int p2p_targets_per_lane, int m2l_waves)
 int sfmm_synchronize(sfmm_plan plan);
 
 /* Device milliseconds of each stage of the last evaluation:
- * [0] gather, [1] P2M, [2] M2M, [3] M2L, [4] L2L, [5] L2P, [6] P2P, [7] scatter, [8] total. */
+ * [0] gather, [1] P2M, [2] M2M, [3] M2L, [4] L2L, [5] L2P, [6] P2P, [7] scatter, [8] total.
+ * Waits for that evaluation, not for later work on the plan's stream.  A stage lasts from
+ * its first kernel's start to the next stage's; the gather and the scatter end
+ * with their last-numbered workgroup, which others may outlast by microseconds. */
 int sfmm_last_stage_ms(sfmm_plan plan, float ms[9]);
 
 /* Records the stage times of each of the next `count` evaluations in a set of its own

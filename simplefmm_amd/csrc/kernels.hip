@@ -46,7 +46,7 @@ __global__ void gather_charges_kernel(int64_t n, int qdim, const int32_t* __rest
     // the block's outputs, which are contiguous
     const int64_t end = min(n, s0 + blockDim.x) * nout;
     for (int64_t i = s0 * nout + threadIdx.x; i < end; i += blockDim.x) out[i] = 0.0;
-    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) stamp[1] = wall_clock64();
+    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) stamp_store(stamp + 1, wall_clock64());
 }
 
 __global__ void stamp_kernel(uint64_t* stamp) { stage_stamp(stamp); }
@@ -56,14 +56,20 @@ __global__ void stamp_kernel(uint64_t* stamp) { stage_stamp(stamp); }
 // order (coalesced read-modify-write) and the sorted side gathered through the
 // inverse permutation.
 __global__ void scatter_outputs_kernel(int64_t n, int nout, const int32_t* __restrict__ iperm,
-                                       const double* __restrict__ out, double* __restrict__ U, uint64_t* stamp)
+                                       const double* __restrict__ out, double* __restrict__ U, uint64_t* stamp,
+                                       uint64_t number)
 {
     stage_stamp(stamp);
     const int64_t o = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (o >= n) return;
     const int64_t s = iperm[o];
     for (int c = 0; c < nout; ++c) U[o * nout + c] += out[s * nout + c];
-    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) stamp[1] = wall_clock64();
+    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        stamp_store(stamp + 1, wall_clock64());
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // in this order
+        __builtin_amdgcn_s_waitcnt(0);
+        stamp_store(stamp + 2, number);
+    }
 }
 
 __global__ void fill_kernel(double* x, int64_t count, double v)
@@ -988,10 +994,11 @@ void launch_stamp(uint64_t* stamp, hipStream_t s)
     if (stamp) hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(64), 0, s, stamp);
 }
 
-void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, uint64_t* stamp, hipStream_t s)
+void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, uint64_t* stamp, uint64_t number,
+                            hipStream_t s)
 {
     hipLaunchKernelGGL(scatter_outputs_kernel, dim3(grid_for(d.n, 256)), dim3(256), 0, s, d.n, nout, d.iperm, out, U,
-                       stamp);
+                       stamp, number);
 }
 
 void launch_fill(double* x, int64_t count, double v, hipStream_t s)

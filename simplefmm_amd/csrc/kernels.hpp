@@ -21,9 +21,14 @@ enum Mode : int {
 // (L2P at p = 16: 95 us, and 120 with it).  Events between the stages held the stream
 // up instead: a 2k evaluation took 75 us with them and takes 37, one of 5k 447 and
 // 405, 20k mixed 387 and 375; no difference from 100k on.  Null: not noted.
+// The stores go to memory: they are read beside later work on the stream.
+__device__ __forceinline__ void stamp_store(uint64_t* p, uint64_t v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 __device__ __forceinline__ void stage_stamp(uint64_t* p)
 {
-    if (p && (blockIdx.x | threadIdx.x) == 0) *p = wall_clock64();
+    if (p && (blockIdx.x | threadIdx.x) == 0) stamp_store(p, wall_clock64());
 }
 
 // Device view of everything a launch needs.  All pointers are device memory.
@@ -186,7 +191,9 @@ constexpr int64_t tr_split_most(int p, bool upper)
 void launch_gather_charges(const DevPlan& d, int qdim, const double* Q, double* q, int nout, double* out, uint64_t* stamp,
                            hipStream_t s);
 void launch_stamp(uint64_t* stamp, hipStream_t s);
-void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, uint64_t* stamp, hipStream_t s);
+// Notes its end at stamp[1] and then the evaluation's number at stamp[2].
+void launch_scatter_outputs(const DevPlan& d, int nout, const double* out, double* U, uint64_t* stamp, uint64_t number,
+                            hipStream_t s);
 void launch_p2m(const DevPlan& d, Mode mode, int nc, const double* q, double* M, hipStream_t s);
 void launch_m2m(const DevPlan& d, LevelSpan parents, int nc, double* M, hipStream_t s);
 void launch_m2l(const DevPlan& d, int nc, const double* M, double* L, hipStream_t s);
