@@ -989,8 +989,9 @@ int run_on(sfmm_plan_s* P, sfmm::Mode mode, int nc, int qdim, const double* dQ, 
                 sfmm::launch_pair_copy(P->M + sp.node0 * nc * P->K, sp.nodes, nc, P->p, P->Mx,
                                        &sp == W.span.data() ? stamp(3) : nullptr, s);
                 sfmm::BcastArgs A = W.args;
-                A.Mx = P->Mx;
-                A.node0 = sp.node0;
+                // as if the copy held every node (an offset in the kernel took 0.7% of it)
+                A.Mx = reinterpret_cast<const double*>(reinterpret_cast<uintptr_t>(P->Mx) -
+                                                       sizeof(double) * sp.node0 * nc * 2 * sfmm::bcast_pairs(P->p));
                 A.item += 4 * sp.item0;
                 A.n_item = sp.items;
                 sfmm::launch_m2l_bcast(A, P->p, nc, P->L, s);
@@ -1596,10 +1597,14 @@ int sfmm_plan_create(sfmm_tree tree, const sfmm_plan_desc* desc, sfmm_plan* out)
     //      and partial-row offsets by prefix sums; then the items in place.
     const int64_t nleaf = static_cast<int64_t>(t.leaf_node.size());
     std::vector<int64_t> near_pref(t.near_begin.size());
-    // A run is one wavefront's work: `most` pairs, a sixteenth of a SIMD's share
-    // of all pairs, so that the last runs end together (an eighth: 200k Plummer
-    // 0.49 ms); a leaf of up to half as much again stays whole (no partial sums).  A source tile takes its latency (LDS, a
-    // tile's fetch) however few targets share it: fewer than 16 count as 16.
+    // A run is one wavefront's work: about `most` pairs (at least a tile of 64
+    // sources), a sixteenth of a SIMD's share of all pairs, so that the last runs end
+    // together (an eighth: 200k Plummer 0.49 ms); a leaf of up to half as much again
+    // stays whole (no partial sums).  A source tile takes its latency (LDS, a tile's
+    // fetch) however few targets share it: fewer than 16 count as 16.  The least limit
+    // is 2^14 pairs once the leaves alone give every SIMD several wavefronts, 2^12
+    // below (near field with 2^12 / 2^14, us: 2k uniform 21 / 45, 20k 41 / 60, 60k 58 / 49,
+    // 100k 107 / 102; 20k Plummer 119 / 104, 60k 224 / 228).
     // (One limit of 2^18 pairs for every tree left a few wavefronts working
     // alone: 200k Plummer, 1 component, 1.70 -> 0.37 ms; 5k uniform, curl, 172 ->
     // 24 us; 20k Plummer mixed 460 -> 105 us; 16M Plummer 14.5 -> 13.9 ms.)
@@ -1943,7 +1948,8 @@ int sfmm_record_stages(sfmm_plan plan, int count)
         plan->rec_count = plan->rec_used = 0;
         const size_t bytes = need * plan->kStamps * sizeof(uint64_t);
         if (dev_malloc(&plan->rec_mem, bytes) != hipSuccess) return fail(SFMM_ERR_ALLOC, "hipMalloc failed (stage times)");
-        HIP_TRY(hipMemcpy(plan->rec_mem, std::vector<uint64_t>(need * plan->kStamps).data(), bytes, hipMemcpyHostToDevice));
+        sfmm::launch_fill(reinterpret_cast<double*>(plan->rec_mem), static_cast<int64_t>(need) * plan->kStamps, 0.0, plan->stream);
+        HIP_TRY(hipGetLastError());
         plan->rec_cap = need;
         for (size_t k = 0; k < need; ++k) plan->rec.push_back({plan->rec_mem + plan->kStamps * k});
     }

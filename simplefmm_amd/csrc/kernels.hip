@@ -46,7 +46,7 @@ __global__ void gather_charges_kernel(int64_t n, int qdim, const int32_t* __rest
     // the block's outputs, which are contiguous
     const int64_t end = min(n, s0 + blockDim.x) * nout;
     for (int64_t i = s0 * nout + threadIdx.x; i < end; i += blockDim.x) out[i] = 0.0;
-    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) stamp_store(stamp + 1, wall_clock64());
+    if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) stamp[1] = wall_clock64();
 }
 
 __global__ void stamp_kernel(uint64_t* stamp) { stage_stamp(stamp); }
@@ -65,10 +65,10 @@ __global__ void scatter_outputs_kernel(int64_t n, int nout, const int32_t* __res
     const int64_t s = iperm[o];
     for (int c = 0; c < nout; ++c) U[o * nout + c] += out[s * nout + c];
     if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-        stamp_store(stamp + 1, wall_clock64());
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // in this order
-        __builtin_amdgcn_s_waitcnt(0);
-        stamp_store(stamp + 2, number);
+        // to memory and in this order: they are read beside later work on the stream
+        __hip_atomic_store(stamp + 1, wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __hip_atomic_store(stamp + 2, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -639,8 +639,9 @@ __device__ __forceinline__ void pair_kernel_f32(float dx, float dy, float dz, co
 }
 
 // Near field (N2N, fmm.hpp:773-809), one wavefront per work item.  An item is
-// a target leaf and a run of its near list, at most a limit of pairs for the tree
-// (the concatenation of its merged source ranges): leaves whose near list is
+// a target leaf and a run of its near list (the concatenation of its merged source
+// ranges), of about the tree's limit of pairs: whole tiles of 64 sources, at least
+// one, and up to 1.5 times the limit where that is the whole list.  Leaves whose near list is
 // long (coarse leaves next to deep subtrees) are split over several items so
 // that no wavefront carries a long tail.  Each lane holds T targets (T = 1, 2
 // or 4, the tile shape: every source read from LDS serves T independent

@@ -19,16 +19,11 @@ enum Mode : int {
 // of its own (launch_stamp) where a stage begins with a heavy one: a store or another
 // branch ahead of the work of P2M, L2P or P2P costs them scalar loads and registers
 // (L2P at p = 16: 95 us, and 120 with it).  Events between the stages held the stream
-// up instead: a 2k evaluation took 75 us with them and takes 37, one of 5k 447 and
-// 405, 20k mixed 387 and 375; no difference from 100k on.  Null: not noted.
-// The stores go to memory: they are read beside later work on the stream.
-__device__ __forceinline__ void stamp_store(uint64_t* p, uint64_t v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
+// up: one event costs 5 us of a 2k evaluation's 74, and there were nine.  Null: not
+// noted.
 __device__ __forceinline__ void stage_stamp(uint64_t* p)
 {
-    if (p && (blockIdx.x | threadIdx.x) == 0) stamp_store(p, wall_clock64());
+    if (p && (blockIdx.x | threadIdx.x) == 0) *p = wall_clock64();
 }
 
 // Device view of everything a launch needs.  All pointers are device memory.
@@ -118,9 +113,9 @@ struct BcastArgs {
     const double* coax = nullptr;        // [28][registers][16] coaxial elements
     const double* az_fwd = nullptr;      // [343][16] (cos m phi - 1, sin m phi), m = 1..16
     const double* az_back = nullptr;     // [343][16] (cos m phi, sin m phi)
-    // multipoles, [gnode - node0][pair (n, m)][nc][Re, Im] (order 0 / sqrt 2) + one zero node; L may be what they were copied from
+    // multipoles, [gnode][pair (n, m)][nc][Re, Im] (order 0 / sqrt 2) + one zero node, of the
+    // gnodes that step_src names (others are not there); L may be what they were copied from
     const double* Mx = nullptr;
-    int64_t node0 = 0;
     const double *rot_sin = nullptr, *coax_sin = nullptr;  // p > 13: rot and coax hold the cos blocks, these the sin
     int64_t n_partial = 0;
     double* partial = nullptr;           // [n_partial, p > 13: cos then sin][(p+1)^2][64]

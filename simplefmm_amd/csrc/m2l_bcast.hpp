@@ -37,6 +37,8 @@
 // (before: one offset at a time, four barriers) 5.03 -> 1.86 ms.  Bound by FP64
 // issue (vector ALU busy 64% of the kernel at p = 12; two wavefronts of a SIMD
 // reach 80%); the rest is waits at the two barriers and for the columns.
+// Registers spilled per lane: p = 12 3, p = 13 48-63, p = 15 9-12 and p = 16 69-93 in
+// the cos kernel (0 and 7-11 in the sin kernel), none at the other orders.
 #pragma once
 
 #include <cstddef>
@@ -57,7 +59,10 @@ constexpr int kBcastMaxP = 16;
 // the first's result) the cos and the sin blocks.  The parts meet only in the
 // azimuths, so they can run apart; both gather all columns then.  Above p = 13 one
 // kernel for both would exceed the registers and the instruction cache
-// (24 sum (n+1)^2 + n^2 bytes of products; 64 KB shared by two compute units).
+// (24 sum (n+1)^2 + n^2 bytes of products; 64 KB shared by two compute units).  At
+// p = 13 two kernels gain with several components and lose with one, whose columns
+// cost most (200k Plummer, one kernel / two: 4 components 3.54 / 2.99 ms, 1 component
+// 1.08 / 1.29).
 enum BcastPart : int { kBcastBoth = 0, kBcastCos = 1, kBcastSin = 2 };
 SFMM_BC_HD constexpr bool bcast_parted(int P) { return P > 13; }
 SFMM_BC_HD constexpr bool bcast_runs_part(int mode, int part)  // part 0 = cos, 1 = sin
@@ -103,7 +108,9 @@ SFMM_BC_HD constexpr int bcast_size(int P, bool coax, int i, int part)
 // index stay together (they share columns and accumulators, or operators)
 // unless the pair exceeds a wavefront's share by a tenth; longest first, then
 // moves and swaps that lower the largest load of a SIMD (wavefronts w, w + 4, ..),
-// of a wavefront, and its registers for columns.
+// of a wavefront, and its registers for columns, weighed 20 : 15 : 3 (the loads of
+// wavefronts alone: 1M Plummer p = 12 11.04 -> 11.12 ms, p = 11 9.05 -> 9.23, 300k p = 6
+// 0.612 -> 0.620, 200k uniform p = 10 curl 0.472 -> 0.481).
 SFMM_BC_HD constexpr BcastUnits bcast_units(int P, bool coax, int mode)
 {
     const int NW = bcast_waves(P), NS = NW < 4 ? NW : 4;
@@ -235,7 +242,10 @@ SFMM_BC_HD constexpr int bcast_resident(int P)
 // Length of the next run when `left` steps of an XCD's share are still to be
 // dealt out: whole groups (up to 189 steps) while there are many left, then ever
 // shorter runs, so that the last workgroups end together.  A run's partial
-// sums cost about 3 steps to write and add, hence the least length.
+// sums cost about 3 steps to write and add, hence the least length, less where even
+// all steps are few (M2L with least 2 / 4 / 8 / 16 steps, us: 2k uniform p = 8 34.6 / 26.9
+// / 29.2 / 41.1; 5k Plummer p = 8 63.4 / 50.5 / 47.8 / 62.0; 20k uniform p = 8 80.8 /
+// 70.9 / 65.5 / 64.4; 20k Plummer p = 12 322 / 313 / 303 / 315).
 inline int64_t bcast_run_steps(int P, int64_t left, int64_t n_step)
 {
     const int64_t r = left * 2 / (3 * 32 * bcast_resident(P)), least = n_step < 2048 ? 4 : 8;

@@ -41,8 +41,10 @@ __host__ __device__ constexpr int row_of(int mode, int n, int m, int part)
 
 // c += op[lane LN of this lane's 16-lane row] * x.  The compiler does not form
 // this instruction from v_mov_b64_dpp and v_fma_f64, hence the asm.  A DPP read
-// needs two wait states after a vector write of op: op comes from memory, and an
-// s_nop at the start of a step separates it from any register copy before.
+// needs two wait states after a vector write of op: op comes from memory, an s_nop
+// separates it from the copies at a change of class, and a test follows every path
+// through the built kernels back from the reads for any copy of the compiler's.  (An
+// s_nop in every step took 0.6% of the M2L: 16M Plummer p = 12 177.8 -> 179.0 ms.)
 template <int LN>
 __device__ __forceinline__ void fmac_row(double& c, double op, double x)
 {
@@ -101,11 +103,10 @@ constexpr ColumnList column_list()
     return c;
 }
 
-// Columns read from LDS ahead of their use (fewer where registers are short).
-
 template <int P, int NC, int MODE, int W>
 struct Wave {
     static constexpr int NW = bcast_waves(P);
+    // columns read from LDS ahead of their use (fewer where registers are short)
     static constexpr int kAheadX = P >= 16 ? 3 : 6;
     static constexpr const BcastUnits& UR = kUnits<P, false, MODE>;
     static constexpr const BcastUnits& UT = kUnits<P, true, MODE>;
@@ -320,7 +321,7 @@ __device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t g, int64_
 #pragma unroll
     for (int k = 0; k < (WV::NCOL > 0 ? WV::NCOL : 1); ++k) wv.are[k] = wv.aim[k] = 0.0;
 
-    const D2* Mx = reinterpret_cast<const D2*>(a.Mx) + comp - a.node0 * (NP * NC);
+    const D2* Mx = reinterpret_cast<const D2*>(a.Mx) + comp;
     // steps are counted from s0 in 32 bits
     const int ns = static_cast<int>(s1 - s0);
     const int32_t* srcs = a.step_src + s0 * (4 * TB) + row * TB + t;
@@ -352,8 +353,8 @@ __device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t g, int64_
                 for (int k = 0; k < WV::NR; ++k)
                     if (st > 0) wv.rot.v[k] = wv.bank.v[k];
                 load_ops<WV::NT>(wv.bank.v, cox_ops(w), lane);
+                asm volatile("s_nop 1");
             }
-            asm volatile("s_nop 1");  // in every step: a copy may end the step before, too
             __builtin_amdgcn_sched_barrier(0);
             change = cls_of(wn) != cls_of(w);
             wv.stage1(X, lane, f.x, f.y);
@@ -424,7 +425,8 @@ __device__ __forceinline__ void bcast_wave(const BcastArgs& a, int64_t g, int64_
             }
         });
     });
-    barrier_lds();    }
+    barrier_lds();
+    }
 }
 
 // L (or, when the group's steps are cut into several runs, the run's partial

@@ -394,12 +394,12 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
     // a wave-uniform float held in a scalar register
     auto uniform = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
 
-    // copies chunks [from, to) of this wavefront's CH / NW chunks of 1 KiB of the
-    // operator of class cls into an LDS buffer
-    auto dma = [&](int cls, dh8* __restrict__ buf, int lane, int from, int to) {
+    // copies this wavefront's CH / NW chunks of 1 KiB of the operator of class cls into
+    // an LDS buffer
+    auto dma = [&](int cls, dh8* __restrict__ buf, int lane) {
         const dh8* src = static_cast<const dh8*>(a.ops) + static_cast<int64_t>(cls) * CH * 64;
 #pragma unroll
-        for (int c = from; c < to; ++c)
+        for (int c = 0; c < CH / NW; ++c)
             dense_lds_copy(src + (w + NW * c) * 64 + lane, buf + (w + NW * c) * 64);
     };
     auto src_ptr = [&](int32_t s) -> const float* {
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
     };
     int32_t src1 = -1;  // this lane's source of the next entry
     if (ne > 0) {
-        dma(a.ent_meta[e0] & 0xff, opbuf0, lane, 0, CH / NW);
+        dma(a.ent_meta[e0] & 0xff, opbuf0, lane);
         const float* csp = src_ptr(a.ent_src[e0 * TB + ti]);
         src1 = a.ent_src[(e0 + (ne > 1 ? 1 : 0)) * TB + ti];
         if (ne < 2) src1 = -1;
@@ -456,8 +456,9 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
         g = __builtin_amdgcn_readfirstlane((smeta[0] >> 8) & 0xff);
         factors(g);
     }
-    // one entry, returning the group of the next (-1: none); even entries read opbuf0 and fill opbuf1, odd ones the reverse
-    // (two arrays, so the reads are seen not to alias the copy in flight)
+    // one entry, returning the group of the next (-1: none); even entries read opbuf0
+    // and fill opbuf1, odd ones the reverse (two arrays, so the reads are seen not to
+    // alias the copy in flight)
     auto entry = [&](const dh8* __restrict__ cur, dh8* __restrict__ nxt) {
         const bool more = i + 1 < ne;
         // the lane and its group, re-read each entry, so that the addresses and the
@@ -474,12 +475,12 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
         dense_wait_all();
         __builtin_amdgcn_s_barrier();
         dense_fence();
-        // The next operator's copy is issued piece by piece between the tiles (all at
-        // once, the wavefronts queue for it before their first products: 1,700 cycles
-        // of an entry's 8,500).  After the last entry once more, unused: a branch
+        // The next operator's copy is issued whole (the wavefronts queue for it before
+        // their first products, 1,700 cycles of an entry's 8,500; spread between the
+        // K-steps it was slower).  After the last entry once more, unused: a branch
         // would make the compiler wait for every load in flight.
         const int ncls = nmeta & 0xff;
-        dma(ncls, nxt, lv, 0, CH / NW);
+        dma(ncls, nxt, lv);
         dense_fence();
         const float* nsp = src_ptr(src1);
         asm volatile("" ::"v"(nsp));  // src1 is used up before its register is loaded again
@@ -502,11 +503,12 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
                 }
             };
             fetch(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, ah, al);
-            // B fragments of a K-step: the columns rotated by e^{i m phi}, scaled and split,
+            // B fragments of a K-step: the columns scaled, rotated by e^{i m phi} and split,
             // slot by slot (the fused products written out, here and in the flush: which
-            // of two products is fused would otherwise change with the code around).  Those of K-step ks + 1 are made between the products of
-            // K-step ks (two sets), in the shadow of the matrix cores; before, all
-            // wavefronts split and then all multiplied.
+            // of two products is fused would otherwise change with the code around).
+            // Those of K-step ks + 1 are made between the products of K-step ks (two
+            // sets), in the shadow of the matrix cores; before, all wavefronts split and
+            // then all multiplied.
             dh8 bch[2], bcl[2], bsh[2], bsl[2];
             auto split = [&](auto kc, auto jc) {
                 constexpr int ks = decltype(kc)::value, j = decltype(jc)::value, B = ks & 1;
