@@ -30,7 +30,8 @@
 //     rounds each earlier contribution once per later group: 3x the error.)
 // Orders 1..12 (the class operator of order 12 fills 66 KiB).
 //
-// 16M Plummer p = 12: 98.2 -> 88.6 ms; 4M uniform p = 10: 27.6 -> 22.4 ms, since
+// 16M Plummer p = 12: 98.2 -> 88.6 ms; 4M uniform p = 10: 27.6 -> 22.4 ms (and 2% more
+// since every column has its own scale), since
 //   * the columns come an offset ahead, the splits move between the products, and
 //     the loop's register copies, which waited for every load in flight, are gone
 //     (93.4 / 25.6);
@@ -521,8 +522,8 @@ __global__ __launch_bounds__(64 * NW, 2) void m2l_dense_kernel(DenseArgs a, cons
                     sm = zq ? 0.0f : sm;
                 }
                 // the scale, a power of two: exact.  (On the columns, 16 multiplies per
-                // K-step and 1% of the evaluation: 4M uniform p = 10 30.7 -> 31.1 ms, 16M
-                // Plummer p = 12 126.0 -> 127.6.  One scale per wavefront would go into
+                // K-step and 1.4-1.8% of the evaluation: 4M uniform p = 10 29.6 -> 30.1 ms,
+                // 16M Plummer p = 12 120.8 -> 122.5.  One scale per wavefront would go into
                 // the azimuth factors.)
                 const float xrj = xr[ks][j] * sc, xij = xi[ks][j] * sc;
                 _Float16 hh, ll;
